@@ -32,6 +32,7 @@
  *                            and its windowed variant), kernels/triton_attention.py:150-202
  *   vrh_paged_decode_noalloc (none: see its declaration)
  *   vrh_paged_prefill        kernels/triton_attention.py:313-366 (paged_prefill_attention)
+ *   vrh_paged_prefill_split_workspace_bytes (none: see its declaration)
  *   vrh_kv_gather            kv_cache_manager.py:834-854 (read)
  *   vrh_kv_finalize          kernels/routing.py:147-177 (finalize_kernel),
  *                            worker/model_runner.py:1331-1346 (its launch)
@@ -167,8 +168,8 @@ int vrh_paged_decode_noalloc(int dtype, void* out, const void* q, const void* ke
  * 16-byte aligned rows) use MFMA tiles with fp32 accumulation; other cases
  * compute each query row with the decode kernel. With a workspace of
  * vrh_paged_prefill_workspace_bytes(num_seqs, max_seqlen_q, q_heads, head_dim)
- * bytes, sequences of one query (decode rows riding in a packed batch) use
- * split-KV decode, and the MFMA work items are dispatched longest sequence
+ * bytes, sequences of one query (decode rows riding in a packed batch of more
+ * than one sequence) use split-KV decode, and the MFMA work items are dispatched longest sequence
  * first (batches of up to 64 sequences are ranked inside the kernel, larger
  * ones up to 2048 by a small ranking kernel writing the order into the
  * workspace). With none (NULL, 0) every sequence goes through the MFMA tiles
@@ -180,6 +181,17 @@ int vrh_paged_decode_noalloc(int dtype, void* out, const void* q, const void* ke
  * n_s - q_s + i + 1 (the decode partition depends only on that length). */
 size_t vrh_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t max_seqlen_q, int32_t q_heads,
                                          int32_t head_dim);
+/* The same workspace plus room for key splits: a call whose query tiles would
+ * leave the GPU partly idle (one prompt chunk, a few short ones) cuts each
+ * tile's keys into up to 16 runs computed side by side and merges their fp32
+ * partials. A call given at least this many bytes does so; with fewer, down to
+ * vrh_paged_prefill_workspace_bytes, it runs one workgroup per tile. The number
+ * of runs follows from the call's shapes, so a query's last bits may differ
+ * between calls of different shapes. */
+size_t vrh_paged_prefill_split_workspace_bytes(int64_t num_seqs, int64_t total_q,
+                                               int32_t max_seqlen_q, int32_t q_heads,
+                                               int32_t kv_heads, int32_t head_dim,
+                                               int32_t block_size, int32_t table_width);
 int vrh_paged_prefill(int dtype, void* out, const void* q, const void* key_cache,
                       const void* value_cache, const int32_t* block_tables,
                       const int32_t* context_lengths, const int32_t* cu_seqlens_q,

@@ -1,0 +1,95 @@
+"""Packed prefill with key splits: calls whose query tiles leave the GPU partly
+idle cut each tile's keys into runs and merge the runs' fp32 partials. Checked
+against the per-query oracle (tolerances of test_gpu_attention) where splitting
+can go wrong: tile and run remainders, tiles shared by a group of q heads that
+does not divide 128, sequences with fewer runs than the longest one, tiles that
+see no key, both grid orders (kv heads a multiple of 8, and not), and partials
+that nothing has initialised.
+"""
+
+import pytest
+import torch
+
+from test_gpu_attention import assert_close, oracle_prefill, prefill_inputs
+
+pytestmark = pytest.mark.gpu
+
+# (context, queries) per sequence; every batch has over 8 queries somewhere, so
+# that it runs on the MFMA tiles, and few enough tiles to be split.
+BATCHES = {
+    "lone_chunk": [(1500, 129)],
+    "lone_short": [(1411, 9)],
+    "one_query_over": [(700, 33), (641, 32)],
+    "ragged": [(1000, 64), (40, 40), (130, 17), (5, 5), (300, 1)],
+    "no_visible_key": [(3, 20), (900, 10)],
+}
+
+
+def call(lib, inputs, nbytes, fill=0xFF):
+    from vllm_rlt.kernels.hip_attention import dtype_code
+
+    q, k, v, tables, lengths, cu, max_q = inputs
+    out = torch.empty_like(q)
+    workspace = torch.full((nbytes,), fill, dtype=torch.uint8, device=q.device)
+    lib.check(lib.vrh_paged_prefill(
+        dtype_code(q.dtype), out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+        tables.data_ptr(), lengths.data_ptr(), cu.data_ptr(), len(lengths), q.shape[0], max_q,
+        q.shape[1], k.shape[2], q.shape[2], k.shape[1], tables.shape[1], tables.stride(0),
+        q.stride(0), q.stride(1), out.stride(0), out.stride(1), *k.stride()[:3], *v.stride()[:3],
+        workspace.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream), "vrh_paged_prefill")
+    return out
+
+
+def sizes(lib, inputs):
+    q, k, _, tables, lengths, _, max_q = inputs
+    base = lib.vrh_paged_prefill_workspace_bytes(len(lengths), max_q, q.shape[1], q.shape[2])
+    full = lib.vrh_paged_prefill_split_workspace_bytes(
+        len(lengths), q.shape[0], max_q, q.shape[1], k.shape[2], q.shape[2], k.shape[1],
+        tables.shape[1])
+    return base, full
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("dtype,heads,kv_heads,head_dim", [
+    (torch.bfloat16, 8, 8, 128), (torch.bfloat16, 12, 4, 128), (torch.float16, 32, 8, 64),
+    (torch.bfloat16, 5, 1, 96), (torch.float16, 2, 2, 32)])
+def test_split_tiles_match_oracle(gpu, batch, dtype, heads, kv_heads, head_dim):
+    from vllm_rlt.kernels._hip import library
+
+    lib = library()
+    inputs = prefill_inputs(BATCHES[batch], heads, kv_heads, head_dim, dtype, gpu, seed=5)
+    base, full = sizes(lib, inputs)
+    assert full > base  # this call splits
+    expected = oracle_prefill(*inputs[:6])
+    # 0xFF bytes are NaN in fp32: a partial read before it is written shows.
+    assert_close(call(lib, inputs, full), expected, dtype)
+    # The smaller workspace of a caller that knows nothing of splits still works.
+    assert_close(call(lib, inputs, base), expected, dtype)
+    assert_close(call(lib, inputs, full - 1), expected, dtype)
+
+
+def test_split_prefill_in_a_graph_follows_the_device_lengths(gpu):
+    """Captured once with wide tables, replayed after the lengths changed: the
+    runs come from the device lengths, the grid only from the shapes."""
+    from vllm_rlt.kernels.hip_attention import paged_prefill_attention
+
+    sequences = [(1400, 100), (60, 30)]
+    q, k, v, tables, lengths, cu, max_q = prefill_inputs(sequences, 8, 8, 128, torch.bfloat16,
+                                                         gpu, seed=9)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        paged_prefill_attention(q, k, v, tables, lengths, cu, max_q)
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = paged_prefill_attention(q, k, v, tables, lengths, cu, max_q)
+    for n in (1400, 131, 100, 1024):
+        lengths[0] = n
+        captured.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, paged_prefill_attention(q, k, v, tables, lengths, cu, max_q))
+        assert_close(captured, oracle_prefill(q, k, v, tables, lengths, cu), torch.bfloat16)

@@ -157,6 +157,31 @@ def test_prefill_workspace_covers_the_decode_rows_it_routes():
             assert pre(seqs, max_q, 16, 128) == need + 4 * seqs
 
 
+def test_prefill_split_workspace_follows_the_shapes():
+    """Room for key splits is asked for only where tiles leave the GPU idle, is
+    bounded, and never falls below the workspace without splits."""
+    lib = _hip.library()
+    pre = lib.vrh_paged_prefill_workspace_bytes
+    split = lib.vrh_paged_prefill_split_workspace_bytes
+
+    def extra(seqs, total, max_q, heads, kv, dim, block, width):
+        both = split(seqs, total, max_q, heads, kv, dim, block, width), pre(seqs, max_q, heads, dim)
+        assert both[0] >= both[1]
+        return both[0] - both[1]
+
+    slot = 128 * 130 * 4
+    assert extra(1, 512, 512, 16, 16, 128, 16, 448) >= 64 * 2 * slot  # one chunk, 7168 keys
+    assert extra(1, 512, 512, 16, 16, 128, 16, 8) == 0                # 128 keys: nothing to cut
+    assert extra(16, 8192, 512, 16, 16, 128, 16, 512) == 0            # 1024 tiles fill the chip
+    assert extra(4, 8, 8, 16, 16, 128, 16, 512) == 0                  # decode rows
+    assert extra(65, 650, 10, 4, 4, 128, 16, 512) == 0                # not ranked in the kernel
+    assert extra(1, 0, 512, 16, 16, 128, 16, 448) == 0
+    for seqs in (1, 2, 7, 64):
+        for total in (9, 100, 1000):
+            for heads, kv in ((16, 16), (32, 8), (5, 1), (64, 4)):
+                assert extra(seqs, total, 512, heads, kv, 128, 16, 2048) <= 1536 * slot + 256
+
+
 def test_library_rejects_bad_arguments_without_a_gpu():
     lib = _hip.library()
     # rows > 0 with a null workspace fails validation before any launch

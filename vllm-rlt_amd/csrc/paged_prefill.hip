@@ -7,8 +7,9 @@
 // dtype before the PV product (as the reference's `weights.to(values.dtype)`).
 //
 // MFMA path (bf16/f16, head_dim a multiple of 32 up to 128):
-//  * Workgroup = 4 waves = 128 query rows of one (sequence, q head); each wave
-//    owns 32 queries. K/V arrive in 32-key sub-blocks staged into LDS (three
+//  * Workgroup = 4 waves = 128 query rows of one (sequence, kv head): query i of
+//    the group's q head g is row i * group + g, so short chunks of grouped-query
+//    heads fill their tiles. Each wave owns 32 rows. K/V arrive in 32-key sub-blocks staged into LDS (three
 //    stages, loaded straight into LDS two sub-blocks ahead) and shared by
 //    the 4 waves; one barrier per sub-block.
 //  * Three workgroups per CU (three waves per SIMD, at most 168 VGPRs): a
@@ -23,6 +24,9 @@
 //    LDS. V stays row-major in LDS; the V^T A-operand comes from two
 //    ds_read_b64_tr_b16 transposed reads whose keys match the P^T k-slots.
 //    Only the pairing of A and B k-slots matters, not the hardware's k order.
+//  * A call with fewer tiles than the chip holds workgroups cuts the tiles'
+//    keys into runs, one workgroup each, and merges the runs' fp32 partials in
+//    a second launch (split_run, paged_prefill_merge_kernel).
 //  * Per-query running max is reduced over the lane pair (l, l ^ 32) each
 //    sub-block; the running sum stays a per-lane partial until the end.
 // Other dtypes / head dims (f32 reference checks, odd dims) run the decode
@@ -54,10 +58,12 @@ constexpr int kBM = kWQ * kWaves;          // queries per workgroup
 constexpr int kSB = 32;                    // keys per sub-block (one pipeline step)
 constexpr int kStages = 3;                 // LDS stages: one sub-block each
 constexpr int kTableSeg = 512;             // page ids staged in LDS at a time
+constexpr int kMinRun = 4;                 // sub-blocks of the shortest key split
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
@@ -94,13 +100,19 @@ struct PrefillArgs {
   int64_t v_block, v_token, v_head;
   int64_t table_stride;
   int64_t num_seqs;
-  int32_t qblocks, kv_heads;
+  int32_t qblocks, kv_heads;  // qblocks: tiles of kBM virtual query rows per (sequence, kv head)
+  int32_t splits;             // key splits per tile (1: none, no partials)
+  int32_t cap_tiles;          // upper bound of the batch's tiles per kv head
+  int32_t target;             // workgroups the key splits aim at
+  float* part_acc;            // [tile, kv head, split][wave][d block][4][64 lanes][4]
+  float* part_ml;             // [tile, kv head, split][wave][32 queries][2]
   int32_t group, block_size, bs_shift, table_width;
   int32_t skip_q;  // sequences with q_len <= skip_q are left to the decode kernel
   int32_t uniform_pages;  // block size a power-of-two multiple of 256 / (16-byte chunks per row)
   int32_t same_kv32;      // K and V block/token strides equal and below 2^31
   const int32_t* order;   // sequences in dispatch order (longest first), or null
   int32_t rank_in_kernel; // num_seqs <= 64: each wave ranks the sequences itself
+  int32_t compact;        // grid over the numbered tiles (rank_in_kernel, kv_heads % 8 == 0)
   float scale_log2;
 };
 
@@ -145,6 +157,62 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* p) {
 constexpr int kWgPerCu = 3;
 constexpr int kWavesPerEu = kWgPerCu * kWaves / 4;
 
+// Batches of up to 64 sequences: every wave ranks them itself, one per lane,
+// longest first (equal lengths in batch order). Tiles (kBM virtual query rows)
+// are numbered in that order, a sequence's last (longest) tile first.
+struct Batch {
+  int q_begin, q_len, n;  // this lane's sequence (0 past the last); n clamped to the table
+  int tiles;              // its tiles per kv head
+  int rank;               // its place in the order
+  int before;             // tiles of the sequences before it
+  // Of the whole batch, per kv head: tiles, their sub-blocks (a tile's keys end
+  // between n - q_len and n; taken as half way), sub-blocks of the longest tile.
+  int all_tiles, work, longest;
+};
+__device__ __forceinline__ Batch rank_batch(const PrefillArgs& a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t cap = (int64_t)a.table_width * a.block_size;
+  Batch b = {};
+  int key = -1;
+  if (lane < a.num_seqs) {
+    b.q_begin = a.cu[lane];
+    b.q_len = a.cu[lane + 1] - b.q_begin;
+    const int len = a.lengths[lane];
+    b.n = (int)(len < 0 ? 0 : ((int64_t)len > cap ? cap : len));
+    if (b.q_len > a.skip_q)
+      b.tiles = (int)min(((int64_t)b.q_len * a.group + kBM - 1) / kBM, (int64_t)a.qblocks);
+    // Distinct keys: one compare per pair below.
+    key = (b.q_len > a.skip_q ? min(b.n, (1 << 24) - 1) + 1 : 0) * 64 + 63 - lane;
+  }
+  const int mine = min(b.tiles * (max(0, b.n - b.q_len / 2) / kSB + 1), 1 << 24);
+  for (int j = 0; j < (int)a.num_seqs; ++j) {
+    const bool ahead = __builtin_amdgcn_readlane(key, j) > key;
+    const int tiles = __builtin_amdgcn_readlane(b.tiles, j);
+    b.rank += ahead;
+    b.before += ahead ? tiles : 0;
+    b.all_tiles += tiles;
+    b.work += __builtin_amdgcn_readlane(mine, j);
+    b.longest = max(b.longest, tiles > 0 ? __builtin_amdgcn_readlane(b.n, j) / kSB + 1 : 0);
+  }
+  return b;
+}
+
+// Key splits: tiles are cut along the keys into runs of this many 32-key
+// sub-blocks, one workgroup per run, so that a call with few tiles still fills
+// the chip and long tiles do not outlast short ones. Worked out from the
+// lengths by every wave, so nothing is read back to the host. One workgroup's
+// step takes ~0.9 us alone on its CU and ~1.0 us with two others beside it, so
+// the runs aim at one full residency of the chip: 512 queries after 6656 keys
+// (16 x 128 heads, 64 tiles) 194 us unsplit, 61 / 56 / 55 / 62 us aiming at 384 /
+// 512 / 768 / 1024 workgroups. Past that the partials cost more than they save
+// (66 KB written and read per workgroup; 6 us of write and a 10 us merge here).
+__device__ __forceinline__ int split_run(const Batch& b, const PrefillArgs& a) {
+  // A tile's last run is shorter: leave room for one such run per tile.
+  const int items = max(a.target - b.all_tiles * a.kv_heads, a.target / 4);
+  const int run = (int)min(((int64_t)b.work * a.kv_heads + items - 1) / items, (int64_t)1 << 24);
+  return max(max(kMinRun, run), ceil_div(b.longest, a.splits));
+}
+
 // Page addressing modes: kDiv (any block size), kShift (power of two).
 enum PageMode { kDiv = 0, kShift = 1 };
 
@@ -168,63 +236,81 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
   const int col = lane & 31;  // query column of this lane
   const int half = lane >> 5; // k-slot half (0 or 1)
   // XCD-aware order: workgroup ids are dealt round-robin to the 8 XCDs (id L
-  // runs on XCD L % 8). A group = one (sequence, kv head); its work items --
-  // every query block of every q head reading that K/V -- all go to XCD
-  // group % 8, back to back, so their K/V tiles are shared in that XCD's L2.
-  // Within a group the longest (last) query blocks run first.
-  const int per_group = a.group * a.qblocks;
-  const int64_t slot = blockIdx.x / 8;
-  const int64_t g = (slot / per_group) * 8 + blockIdx.x % 8;
-  if (g >= a.num_seqs * a.kv_heads) return;
-  const int r_item = (int)(slot % per_group);
-  const int head = (int)(g % a.kv_heads) * a.group + r_item / a.qblocks;
-  const int qb = a.qblocks - 1 - r_item % a.qblocks;
-  const int kvh = head / a.group;
+  // runs on XCD L % 8), and all tiles of one (sequence, kv head, key split)
+  // should run on one XCD, back to back, so that its L2 serves their K/V.
+  // Splits are outermost: how many of them a tile uses is only known here, and
+  // the unused ones must not thin out some XCDs more than others.
   const int64_t cap = (int64_t)a.table_width * a.block_size;
   int64_t seq;
-  int q_begin, q_len, n;
+  int q_begin, q_len, n, kvh, qb, split = 0;
+  int tile = 0;       // tile number of the partials
+  int run = 1 << 24;  // sub-blocks of one key split
   if (a.rank_in_kernel) {
-    // Up to 64 sequences: every wave ranks them itself (one lane per
-    // sequence, the same longest-first stable order as prefill_order_kernel)
-    // and takes the sequence of rank g / kv_heads, without a separate launch.
-    const int s = lane;
-    int c0 = 0, c1 = 0, len = 0, key = INT32_MIN;
-    if (s < a.num_seqs) {
-      c0 = a.cu[s];
-      c1 = a.cu[s + 1];
-      len = a.lengths[s];
-      key = c1 - c0 <= a.skip_q ? -1 : (int)(len < 0 ? 0 : ((int64_t)len > cap ? cap : len));
+    const Batch b = rank_batch(a);
+    uint64_t hit;
+    if (a.compact) {
+      // kv_heads a multiple of 8: kv heads fastest over the numbered tiles, so
+      // a kv head's tiles share XCD kvh % 8 and no workgroup is launched for
+      // tiles that shorter sequences do not have.
+      const int per_split = a.cap_tiles * a.kv_heads;
+      split = a.splits > 1 ? (int)(blockIdx.x / per_split) : 0;
+      const int item = (int)blockIdx.x - split * per_split;
+      tile = item / a.kv_heads;
+      kvh = item - tile * a.kv_heads;
+      hit = __ballot(tile >= b.before && tile < b.before + b.tiles);
+    } else {
+      const int64_t slot = blockIdx.x / 8;
+      const int64_t gs = (slot / a.qblocks) * 8 + blockIdx.x % 8;
+      const int64_t groups = a.num_seqs * a.kv_heads;
+      split = a.splits > 1 ? (int)(gs / groups) : 0;
+      const int64_t g = gs - split * groups;
+      kvh = (int)(g % a.kv_heads);
+      tile = (int)(slot % a.qblocks);
+      hit = __ballot(b.rank == (int)(g / a.kv_heads) && tile < b.tiles);
     }
-    int rank = 0;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      const int other = __builtin_amdgcn_readlane(key, j);
-      rank += (other > key) || (other == key && j < s);
-    }
-    const uint64_t hit = __ballot(rank == (int)(g / a.kv_heads) && s < a.num_seqs);
+    if (hit == 0 || split >= a.splits) return;
     const int pick = __builtin_ffsll((long long)hit) - 1;
     seq = pick;
-    q_begin = __builtin_amdgcn_readlane(c0, pick);
-    q_len = __builtin_amdgcn_readlane(c1, pick) - q_begin;
-    n = __builtin_amdgcn_readlane(len, pick);
+    q_begin = __builtin_amdgcn_readlane(b.q_begin, pick);
+    q_len = __builtin_amdgcn_readlane(b.q_len, pick);
+    n = __builtin_amdgcn_readlane(b.n, pick);
+    const int before = __builtin_amdgcn_readlane(b.before, pick);
+    if (!a.compact) tile += before;
+    qb = __builtin_amdgcn_readlane(b.tiles, pick) - 1 - (tile - before);
+    if (a.splits > 1) run = split_run(b, a);
   } else {
+    const int64_t slot = blockIdx.x / 8;
+    const int64_t g = (slot / a.qblocks) * 8 + blockIdx.x % 8;
+    if (g >= a.num_seqs * a.kv_heads) return;
+    kvh = (int)(g % a.kv_heads);
+    qb = a.qblocks - 1 - (int)(slot % a.qblocks);
     seq = a.order ? a.order[g / a.kv_heads] : g / a.kv_heads;
     q_begin = a.cu[seq];
     q_len = a.cu[seq + 1] - q_begin;
     n = a.lengths[seq];
+    n = n < 0 ? 0 : ((int64_t)n > cap ? (int)cap : n);
+    if ((int64_t)qb * kBM >= (int64_t)q_len * a.group || q_len <= a.skip_q) return;
   }
-  if (qb * kBM >= q_len || q_len <= a.skip_q) return;
-  n = n < 0 ? 0 : ((int64_t)n > cap ? (int)cap : n);
   const int prefix = n - q_len;
-  const int qi0 = qb * kBM + wave * kWQ;        // this wave's first query
-  const int qi = qi0 + col;                     // this lane's query
+  // Virtual query row v of the tile: query v / group of the kv head's q head
+  // v % group, so a tile is filled by all the heads that read the same K/V.
+  const int v0 = qb * kBM + wave * kWQ;         // this wave's first row
+  const int qi = (v0 + col) / a.group;          // this lane's query
+  const int head = kvh * a.group + (v0 + col) - qi * a.group;
   const bool q_ok = qi < q_len;
   const int qpos = prefix + qi;
-  const int wave_qpos0 = prefix + qi0;
-  const int end = max(0, min(n, prefix + (qb + 1) * kBM));
-  const int nsub = (end + kSB - 1) / kSB;       // sub-blocks staged by the workgroup
+  const int wave_q0 = v0 / a.group;             // this wave's first query
+  const int wave_qpos0 = prefix + wave_q0;
+  const int end = max(0, min(n, prefix + (qb * kBM + kBM - 1) / a.group + 1));
+  // Sub-blocks [j0, nsub) are this workgroup's share of the tile's keys.
+  const int tile_sub = (end + kSB - 1) / kSB;
+  const int j0 = split * run;
+  const int nsub = min(tile_sub, j0 + run);
+  if (j0 >= nsub && split > 0) return;
   // Sub-blocks this wave computes: keys up to its last query's position.
-  const int nsub_w = qi0 >= q_len ? 0 : (max(0, min(end, wave_qpos0 + kWQ)) + kSB - 1) / kSB;
+  const int nsub_w = wave_q0 >= q_len
+                         ? 0
+                         : (max(0, min(end, prefix + (v0 + kWQ - 1) / a.group + 1)) + kSB - 1) / kSB;
   const int32_t* table = a.tables + seq * a.table_stride;
 
   // Q^T B-operands: lane holds query `col`, dims 16c + 8*half .. +8.
@@ -268,7 +354,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
     if constexpr (MODE == kDiv) return pos / a.block_size;
     else return pos >> a.bs_shift;
   };
-  load_table(0);
+  load_table(page_of(j0 * kSB));
 
   // Sub-block `j` of K/V goes from the pages straight into an LDS stage.
   // Staging instruction r of this wave fills slots 64 * (wave + 4r) .. + 63 of
@@ -534,9 +620,9 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
     if (full_share) vm_wait<kDmaPerStep>();
     else vm_wait<2 * (NI - 1)>();
   };
-  if (nsub > 0) {
-    dma(0, H0{});
-    if (nsub > 1) dma(1, H1{});
+  if (j0 < nsub) {
+    dma(j0, H0{});
+    if (j0 + 1 < nsub) dma(j0 + 1, H1{});
     auto step = [&](int j, auto hc) {
       constexpr int h = decltype(hc)::value;
       using Hd = std::integral_constant<int, (h + 2) % kStages>;
@@ -583,7 +669,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
         acc[i % DB] = Mfma<T>::run(vop[i], pop[i / DB], acc[i % DB]);
       }
     };
-    for (int j = 0; j < nsub; j += kStages) {
+    for (int j = j0; j < nsub; j += kStages) {
       step(j, H0{});
       if (j + 1 >= nsub) break;
       step(j + 1, H1{});
@@ -592,6 +678,25 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
     }
   }
   lsum += shfl_xor_f32(lsum, 32);
+  if (tile_sub > run) {
+    // This split's (m, l, O) in the accumulator's own layout (1 KiB per wave
+    // store); paged_prefill_merge_kernel reads it back the same way.
+    if (wave_q0 >= q_len || tile >= a.cap_tiles) return;
+    const int64_t slot_id = ((int64_t)tile * a.kv_heads + kvh) * a.splits + split;
+    f32x4* dst = reinterpret_cast<f32x4*>(a.part_acc) + (slot_id * kWaves + wave) * DB * 256 + lane;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi)
+        dst[(db * 4 + gi) * 64] = f32x4{acc[db][4 * gi], acc[db][4 * gi + 1], acc[db][4 * gi + 2],
+                                        acc[db][4 * gi + 3]};
+    if (half == 0) {
+      float* ml = a.part_ml + ((slot_id * kWaves + wave) * kWQ + col) * 2;
+      ml[0] = m;
+      ml[1] = lsum;
+    }
+    return;
+  }
   if (!q_ok) return;
   const float inv = fast_rcp(fmaxf(lsum, 1e-30f));
   T* op = reinterpret_cast<T*>(a.out) + (int64_t)(q_begin + qi) * a.o_token + head * a.o_head;
@@ -604,6 +709,92 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
           u32x2{pack2<T>(acc[db][4 * gi] * inv, acc[db][4 * gi + 1] * inv),
                 pack2<T>(acc[db][4 * gi + 2] * inv, acc[db][4 * gi + 3] * inv)};
     }
+  }
+}
+
+// Log-sum-exp merge of a tile's key splits, in split order. One workgroup per
+// (32 query rows, 32 dims) of a tile, one wave per 8 dims: every load is 1 KiB
+// contiguous, and kAhead splits' loads are in flight together.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void paged_prefill_merge_kernel(PrefillArgs a) {
+  constexpr int DB = D / 32;
+  constexpr int kAhead = 4;
+  const int lane = threadIdx.x & 63;
+  const int gi = threadIdx.x >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const int db = blockIdx.x % DB;
+  const int wave = blockIdx.x / DB % kWaves;  // the tile's 32-row group
+  const int tile = blockIdx.x / (DB * kWaves) / a.kv_heads;
+  const int kvh = blockIdx.x / (DB * kWaves) % a.kv_heads;
+  const Batch b = rank_batch(a);
+  const uint64_t hit = __ballot(tile >= b.before && tile < b.before + b.tiles);
+  if (hit == 0) return;
+  const int pick = __builtin_ffsll((long long)hit) - 1;
+  const int q_begin = __builtin_amdgcn_readlane(b.q_begin, pick);
+  const int q_len = __builtin_amdgcn_readlane(b.q_len, pick);
+  const int n = __builtin_amdgcn_readlane(b.n, pick);
+  const int qb = __builtin_amdgcn_readlane(b.tiles, pick) - 1 -
+                 (tile - __builtin_amdgcn_readlane(b.before, pick));
+  const int v0 = qb * kBM + wave * kWQ;
+  if (v0 / a.group >= q_len) return;
+  const int end = max(0, min(n, n - q_len + (qb * kBM + kBM - 1) / a.group + 1));
+  const int active = ceil_div((end + kSB - 1) / kSB, split_run(b, a));
+  if (active <= 1) return;  // written by the tile itself
+  const int64_t slot_id = ((int64_t)tile * a.kv_heads + kvh) * a.splits;
+  const int64_t ml_step = kWaves * kWQ, acc_step = (int64_t)kWaves * DB * 256;
+  const f32x2_t* ml =
+      reinterpret_cast<const f32x2_t*>(a.part_ml) + (slot_id * kWaves + wave) * kWQ + col;
+  const f32x4* src = reinterpret_cast<const f32x4*>(a.part_acc) +
+                     (((slot_id * kWaves + wave) * DB + db) * 4 + gi) * 64 + lane;
+  float M = -1e30f, L = 0.f;
+  f32x4 acc = {};
+  for (int s0 = 0; s0 < active; s0 += kAhead) {
+    f32x2_t w[kAhead];
+    f32x4 v[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int s = min(s0 + u, active - 1);
+      w[u] = ml[s * ml_step];
+      v[u] = src[s * acc_step];
+    }
+    float top = M;
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) top = fmaxf(top, w[u][0]);
+    const float corr = fast_exp2(M - top);
+    M = top;
+    L *= corr;
+    acc *= corr;
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const float x = s0 + u < active ? fast_exp2(w[u][0] - M) : 0.f;
+      if (s0 + u < active) L = fmaf(x, w[u][1], L);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (s0 + u < active) acc[e] = fmaf(x, v[u][e], acc[e]);
+    }
+  }
+  const int qi = (v0 + col) / a.group;
+  if (qi >= q_len) return;
+  const float inv = fast_rcp(fmaxf(L, 1e-30f));
+  T* op = reinterpret_cast<T*>(a.out) + (int64_t)(q_begin + qi) * a.o_token +
+          (int64_t)(kvh * a.group + v0 + col - qi * a.group) * a.o_head + 32 * db + 8 * gi + 4 * half;
+  *reinterpret_cast<u32x2*>(op) =
+      u32x2{pack2<T>(acc[0] * inv, acc[1] * inv), pack2<T>(acc[2] * inv, acc[3] * inv)};
+}
+
+template <typename T>
+bool launch_prefill_merge(int d, dim3 grid, hipStream_t s, const PrefillArgs& a) {
+  switch (d) {
+#define VRH_D(DV)                                                                               \
+  case DV:                                                                                      \
+    hipLaunchKernelGGL((paged_prefill_merge_kernel<T, DV>), grid, dim3(256), 0, s, a);          \
+    return true;
+    VRH_D(32)
+    VRH_D(64)
+    VRH_D(96)
+    VRH_D(128)
+#undef VRH_D
+    default: return false;
   }
 }
 
@@ -691,6 +882,66 @@ extern "C" size_t vrh_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t ma
          (size_t)num_seqs * sizeof(int32_t);
 }
 
+// Key splits of a call whose tiles would leave the chip partly idle. The grid
+// depends on shapes only (graph capture): the tiles are estimated from total_q
+// (a ragged sequence fills half of its last tile on average) and the longest
+// context from the table width; the kernel then sizes the runs from the device
+// lengths (split_plan).
+namespace {
+// Workgroups the splits aim at: those the chip holds at once (256 CUs, three
+// per CU by registers and LDS at head_dim 96 and 128, four at 64 and 32).
+constexpr int kCus = 256;
+int target_items(int32_t head_dim) { return kCus * (head_dim <= 64 ? 4 : kWgPerCu); }
+constexpr int kMaxSlots = 1536;     // partials held (68 KB each at head_dim 128)
+constexpr int kMaxKeySplits = 16;
+// Sub-blocks that splitting must take off the longest tile to pay for the merge
+// launch and the partials: 4 chunks of up to 512 queries without a prefix (16
+// sub-blocks, 416 tiles) took 36 us split in two against 26 us whole, one such
+// chunk (64 tiles) 18.1 against 19.5 us.
+constexpr int kMinSaved = 12;
+
+// Upper bound of the tiles per kv head of a batch whose sequences' query counts
+// sum to at most total_q, each at most max_seqlen_q.
+int64_t most_tiles(int64_t num_seqs, int64_t total_q, int32_t max_seqlen_q, int64_t group) {
+  const int64_t rows = std::min<int64_t>(total_q, num_seqs * max_seqlen_q) * group;
+  return std::min(num_seqs * ceil_div64((int64_t)max_seqlen_q * group, kBM),
+                  (rows + num_seqs * (kBM - 1)) / kBM);
+}
+
+// Most key splits of a tile (1: none).
+int32_t most_splits(int64_t num_seqs, int64_t total_q, int32_t max_seqlen_q, int32_t q_heads,
+                    int32_t kv_heads, int32_t head_dim, int32_t block_size, int32_t table_width) {
+  if (num_seqs < 1 || num_seqs > 64 || total_q < 1 || max_seqlen_q <= kExactQ || kv_heads < 1 ||
+      block_size < 1)
+    return 1;
+  const int64_t group = q_heads / kv_heads;
+  const int64_t most = most_tiles(num_seqs, total_q, max_seqlen_q, group) * kv_heads;
+  // A ragged sequence fills half of its last tile on average.
+  const int64_t est =
+      std::min(most, (total_q * group + num_seqs * kBM / 2) / kBM * kv_heads);
+  const int64_t nsub = ceil_div64((int64_t)table_width * block_size, kSB);
+  const int64_t target = target_items(head_dim);
+  if (est >= target || nsub * (target - est) < kMinSaved * target) return 1;
+  return (int32_t)std::max<int64_t>(
+      1, std::min({(int64_t)kMaxKeySplits, kMaxSlots / most, ceil_div64(nsub, kMinRun)}));
+}
+
+size_t split_slot_bytes(int32_t head_dim) { return (size_t)kBM * (head_dim + 2) * sizeof(float); }
+}  // namespace
+
+extern "C" size_t vrh_paged_prefill_split_workspace_bytes(int64_t num_seqs, int64_t total_q,
+                                                          int32_t max_seqlen_q, int32_t q_heads,
+                                                          int32_t kv_heads, int32_t head_dim,
+                                                          int32_t block_size, int32_t table_width) {
+  const size_t base = vrh_paged_prefill_workspace_bytes(num_seqs, max_seqlen_q, q_heads, head_dim);
+  const int32_t splits = most_splits(num_seqs, total_q, max_seqlen_q, q_heads, kv_heads, head_dim,
+                                     block_size, table_width);
+  if (splits <= 1) return base;
+  return (base + 255) / 256 * 256 +
+         (size_t)most_tiles(num_seqs, total_q, max_seqlen_q, q_heads / kv_heads) * kv_heads * splits *
+             split_slot_bytes(head_dim);
+}
+
 extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void* key_cache,
                                  const void* value_cache, const int32_t* block_tables,
                                  const int32_t* context_lengths, const int32_t* cu_seqlens_q,
@@ -741,7 +992,7 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
   }
   VRH_CHECK_ARG(max_seqlen_q >= 1, "vrh_paged_prefill: max_seqlen_q must be positive");
   VRH_CHECK_ARG(q_heads <= 65535, "vrh_paged_prefill: too many heads");
-  PrefillArgs a;
+  PrefillArgs a = {};  // pointers not set below are null
   a.out = out;
   a.q = q;
   a.k = key_cache;
@@ -764,7 +1015,10 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
   a.block_size = block_size;
   a.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
   a.table_width = table_width;
-  a.skip_q = route_decode ? route_q : 0;
+  // A lone sequence with more than kExactQ queries needs no decode launch: the
+  // tiles handle it whatever its query count turns out to be.
+  const bool route_rows = route_decode && !(num_seqs == 1 && max_seqlen_q > kExactQ);
+  a.skip_q = route_rows ? route_q : 0;
   {
     // Rows one staging instruction covers: 64 lanes of 16 bytes over rows of
     // head_dim / 8 chunks; the fast addressing needs them on one page.
@@ -779,11 +1033,34 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
   a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)head_dim));
   a.num_seqs = num_seqs;
   a.kv_heads = kv_heads;
-  a.qblocks = ceil_div(max_seqlen_q, kBM);
-  a.order = nullptr;
+  const int64_t qblocks = ceil_div64((int64_t)max_seqlen_q * a.group, kBM);
+  VRH_CHECK_ARG(qblocks < (1 << 24), "vrh_paged_prefill: too many work items");
+  a.qblocks = (int32_t)qblocks;
   // Up to 64 sequences are ranked inside the kernel (also without a
   // workspace); larger batches use the ordering kernel and the workspace.
+  a.order = nullptr;
   a.rank_in_kernel = num_seqs > 1 && num_seqs <= 64;
+  // Key splits when the workspace has room for their partials (after the
+  // decode partials and the dispatch order).
+  a.splits = 1;
+  const int64_t cap_tiles = most_tiles(num_seqs, total_q, max_seqlen_q, a.group);
+  a.cap_tiles = (int32_t)std::min<int64_t>(cap_tiles, 1 << 30);
+  a.target = target_items(head_dim);
+  a.part_acc = a.part_ml = nullptr;
+  if (route_decode) {
+    const size_t base =
+        (vrh_paged_prefill_workspace_bytes(num_seqs, max_seqlen_q, q_heads, head_dim) + 255) / 256 * 256;
+    const int32_t splits = most_splits(num_seqs, total_q, max_seqlen_q, q_heads, kv_heads, head_dim,
+                                       block_size, table_width);
+    const size_t slots = (size_t)cap_tiles * kv_heads * splits;
+    if (splits > 1 && workspace_bytes >= base + slots * split_slot_bytes(head_dim)) {
+      a.splits = splits;
+      a.rank_in_kernel = 1;  // the runs follow from the same per-lane lengths
+      a.part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + base);
+      a.part_ml = a.part_acc + slots * kBM * head_dim;
+    }
+  }
+  a.compact = a.rank_in_kernel && kv_heads % 8 == 0;
   // With every sequence routed to the decode kernel (max_seqlen_q <= the
   // routed query count) the MFMA launch, and its ordering, would have no work.
   const bool mfma_work = a.skip_q < max_seqlen_q;
@@ -795,16 +1072,22 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
                        (int64_t)table_width * block_size, order);
     a.order = order;
   }
-  const int64_t groups = num_seqs * kv_heads;
-  const int64_t launched = (groups + 7) / 8 * 8 * (int64_t)a.group * a.qblocks;
+  const int64_t groups = num_seqs * kv_heads * a.splits;
+  const int64_t launched = a.compact ? cap_tiles * kv_heads * a.splits
+                                     : (groups + 7) / 8 * 8 * (int64_t)a.qblocks;
   VRH_CHECK_ARG(launched < (1ll << 31), "vrh_paged_prefill: too many work items");
   if (mfma_work) {
     const bool ok = dtype == VRH_DTYPE_BF16
                         ? launch_prefill<bf16_t>(head_dim, dim3((unsigned)launched), s, a)
                         : launch_prefill<f16_t>(head_dim, dim3((unsigned)launched), s, a);
     VRH_CHECK_ARG(ok, "vrh_paged_prefill: no kernel for head_dim %d", head_dim);
+    if (a.splits > 1) {
+      const dim3 mgrid((unsigned)(head_dim / 32 * kWaves * cap_tiles * kv_heads));
+      if (dtype == VRH_DTYPE_BF16) launch_prefill_merge<bf16_t>(head_dim, mgrid, s, a);
+      else launch_prefill_merge<f16_t>(head_dim, mgrid, s, a);
+    }
   }
-  if (route_decode) {
+  if (route_rows) {
     // Short sequences of the packed batch: one split-KV decode row per query
     // (row r is query r % route_q of sequence r / route_q).
     const int rc = vrh_decode_rows(

@@ -56,6 +56,9 @@ SIGNATURES: dict[str, tuple[object, list]] = {
          _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _SZ, _P],
     ),
     "vrh_paged_prefill_workspace_bytes": (_SZ, [_I64, _I32, _I32, _I32]),
+    "vrh_paged_prefill_split_workspace_bytes": (
+        _SZ, [_I64, _I64, _I32, _I32, _I32, _I32, _I32, _I32]
+    ),
     "vrh_kv_gather": (_INT, [_P, _P, _P, _P, _P, _I64, _I32, _I64, _I64, _I64, _P]),
     "vrh_kv_finalize": (
         _INT, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _P]

@@ -172,8 +172,9 @@ def paged_prefill_attention(q, key_cache, value_cache, block_tables, context_len
         return output
     cu_seqlens_q = cu_seqlens_q.contiguous()
     lib = library()
-    nbytes = lib.vrh_paged_prefill_workspace_bytes(sequences, int(max_seqlen_q), q.shape[1],
-                                                   q.shape[2])
+    nbytes = lib.vrh_paged_prefill_split_workspace_bytes(
+        sequences, q.shape[0], int(max_seqlen_q), q.shape[1], key_cache.shape[2], q.shape[2],
+        key_cache.shape[1], block_tables.shape[1])
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
     lib.check(
         lib.vrh_paged_prefill(
