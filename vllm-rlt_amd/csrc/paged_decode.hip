@@ -11,10 +11,16 @@
 //    or 2 grouped-query heads when they divide the group (each loaded K/V
 //    vector serves all of them), else 1. Groups of 8-16 heads, and of 3, 5, 6
 //    or 7, run on the MFMA kernel below instead (one wave per kv head). A split is a run of whole
-//    pages: bps = max(min_bps, ceil(pages / kMaxSplits)) pages (at least 128
-//    tokens, at most 16 splits per row), so the partition depends only on
+//    pages: bps = max(min_bps, ceil(pages / kMaxSplits)) pages (at least 64
+//    tokens of a 16-bit type, 32 of fp32, at most 16 splits per row), so the partition depends only on
 //    the row's own length -> batch invariance. The split index is rotated
 //    per (row, head) so that every XCD receives the same share of splits.
+//  * A longer split is a chain of up to 8 parts (4 in the MFMA kernel), folded in
+//    order. One wave runs them one after another where the launch has waves
+//    enough; launches of few splits give each split a workgroup with one wave
+//    per part, folded through LDS in the same order: the same bits, many times
+//    the loads in flight. One row of 24001 tokens (16 x 128 heads, bf16) takes
+//    41 us instead of 78, two rows of 32 over 8 heads at 30000 42 instead of 119.
 //  * Lane layout: LPT lanes cover one token's head_dim with VEC elements each
 //    (16-byte global loads for bf16 D=128: LPT=16), so one wave-wide load
 //    instruction fetches TPL = 64 / LPT tokens; U loads of K and U of V are
@@ -42,11 +48,30 @@ namespace {
 // Wave loads per chunk (in flight per lane for each of K and V), minimum and
 // maximum split length, grouped-query heads one wave may serve.
 constexpr int kMaxSplits = 16;
-constexpr int kSplitTokens = 128;  // minimum tokens per split (whole pages)
+// Minimum K bytes of a split (64 tokens of a 16-bit type at head_dim 128, 32 of
+// fp32), at most kSplitTokens tokens (shorter ones of head_dim 64: 18 rows of up
+// to 1757 tokens over 8 kv heads 32 against 24 us). Against 128 tokens of any type: 8 fp32 rows of
+// 64-512 tokens 14.9 against 19.4 us, 64 bf16 rows 36.6 against 39.1, 37 f16
+// rows of up to 6000 over 8 kv heads 103 against 108, 64 rows of 512-4096 the
+// same; 32 tokens of a 16-bit type were slower again (100 rows of up to 300
+// tokens 32.9 against 28.2).
+constexpr int kSplitBytes = 16384;
+constexpr int kSplitTokens = 128;
+constexpr int kParts = 8;           // most parts of a split (VALU kernel, MFMA kernel)
+constexpr int kMfmaParts = 4;
 constexpr int kMaxHpw = 8;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-
 constexpr int kU = 8;                // wave loads per chunk (K and V each)
+
+// d + a.lo * b.lo + a.hi * b.hi of packed 16-bit pairs, in fp32.
+template <typename T>
+__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float d) {
+  if constexpr (std::is_same<T, bf16_t>::value)
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a),
+                                           __builtin_bit_cast(bf16x2_t, b), d, false);
+  else
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b), d,
+                                  false);
+}
 
 template <typename T, int VEC>
 __device__ __forceinline__ typename Vec<T, VEC>::raw_t load_kv(const T* p) {
@@ -81,6 +106,9 @@ struct DecodeArgs {
   int32_t num_seqs;
   int32_t expand_e;
   int32_t q_heads, group, head_dim, block_size, bs_shift, window, min_bps, table_width;
+  int32_t long_bps;   // pages of the shortest split of rows past kMaxSplits shortest splits
+  int32_t min_part;   // pages of the shortest part of a split
+  int32_t max_parts;  // most parts of a split
   float scale_log2;
 };
 
@@ -90,6 +118,7 @@ struct Partition {
   int pages;    // pages touched
   int bps;      // pages per split
   int nsplit;
+  int pps;      // pages per part of a split
 };
 
 __device__ __forceinline__ Partition partition(int n, const DecodeArgs& a) {
@@ -102,8 +131,10 @@ __device__ __forceinline__ Partition partition(int n, const DecodeArgs& a) {
     p.first = p.start / a.block_size;
     p.pages = (n + a.block_size - 1) / a.block_size - p.first;
   }
-  p.bps = max(a.min_bps, ceil_div(p.pages, kMaxSplits));
+  p.bps = max(p.pages <= kMaxSplits * a.min_bps ? a.min_bps : a.long_bps,
+              ceil_div(p.pages, kMaxSplits));
   p.nsplit = ceil_div(p.pages, p.bps);
+  p.pps = min(p.bps, max(a.min_part, ceil_div(p.bps, a.max_parts)));
   return p;
 }
 
@@ -157,14 +188,54 @@ __device__ __forceinline__ int wave_max_i(int x) {
              max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
 }
 
+// A wave's online-softmax state in LDS (one lane's values 64 floats apart).
+template <int HPW, int VEC>
+__device__ __forceinline__ void store_state(float* lds, int lane, const float (&m)[HPW],
+                                            const float (&l)[HPW], const float (&acc)[HPW][VEC]) {
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    float* p = lds + h * (VEC + 2) * 64 + lane;
+    p[0] = m[h];
+    p[64] = l[h];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) p[(2 + i) * 64] = acc[h][i];
+  }
+}
+
+// Combines the state in LDS with the one in registers, into registers. The
+// state of the earlier tokens is the one in LDS when lds_first, so both ways of
+// folding do the same arithmetic.
+template <int HPW, int VEC>
+__device__ __forceinline__ void fold_state(const float* lds, int lane, float (&m)[HPW],
+                                           float (&l)[HPW], float (&acc)[HPW][VEC], bool lds_first) {
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    const float* p = lds + h * (VEC + 2) * 64 + lane;
+    const float mo = p[0], lo = p[64];
+    const float top = fmaxf(m[h], mo);
+    const float safe = top == -INFINITY ? 0.f : top;
+    const float wr = fast_exp2(m[h] - safe), wo = fast_exp2(mo - safe);
+    const float w0 = lds_first ? wo : wr, w1 = lds_first ? wr : wo;
+    m[h] = top;
+    l[h] = fmaf(lds_first ? l[h] : lo, w1, (lds_first ? lo : l[h]) * w0);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const float o = p[(2 + i) * 64];
+      acc[h][i] = fmaf(lds_first ? acc[h][i] : o, w1, (lds_first ? o : acc[h][i]) * w0);
+    }
+  }
+}
+
 // The work of one row and HPW consecutive q heads of one kv head (the
 // grouped-query heads that share it) over splits split0, split0 + step, ...
 // of the row's partition: each K/V vector a lane loads serves all HPW heads.
 // Multi-split rows write (m, l, acc) partials, single splits the output; a
 // zero-length row writes zeros (from split 0).
-template <typename T, int VEC, int LPT, int HPW>
+// WAVES: 0 when no split has more than one part, 1 for parts one after another,
+// else the waves of the workgroup that runs them side by side.
+template <typename T, int VEC, int LPT, int HPW, int WAVES>
 __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, int head0,
-                                            int split0, int step) {
+                                            int split0, int step, float* lds) {
   // Loads per chunk: fewer when many heads' state shares the registers.
   constexpr int U = (2 * kU / HPW) < 1 ? 1 : ((2 * kU / HPW) > kU ? kU : 2 * kU / HPW);
   constexpr int TPL = 64 / LPT;  // tokens per wave load
@@ -172,6 +243,7 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
   using raw_t = typename Vec<T, VEC>::raw_t;
 
   const int lane = threadIdx.x & 63;
+  const int wave = WAVES > 1 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int dg = lane % LPT;
   const int tg = lane / LPT;
   const int kvh = head0 / a.group;
@@ -182,7 +254,7 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
   T* out = reinterpret_cast<T*>(a.out) + qrow * a.o_row + (int64_t)head0 * a.o_head + dg * VEC;
 
   if (n == 0) {
-    if (split0 == 0 && tg == 0 && dvalid) {
+    if (split0 == 0 && wave == 0 && tg == 0 && dvalid) {
       float z[VEC];
 #pragma unroll
       for (int i = 0; i < VEC; ++i) z[i] = 0.f;
@@ -193,10 +265,10 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
   }
   const Partition P = partition(n, a);
   if (split0 >= P.nsplit) return;
-  // bf16 with 8-element vectors: the q.k product runs on packed bf16 pairs
+  // 16-bit types with 8-element vectors: the q.k product runs on packed pairs
   // (v_dot2 with fp32 accumulation, products exact in fp32) against the
   // unscaled q; the scale is applied to the reduced score.
-  constexpr bool kDot2 = std::is_same<T, bf16_t>::value && VEC == 8;
+  constexpr bool kDot2 = sizeof(T) == 2 && VEC == 8;
   uint32_t qp2[HPW][VEC / 2];
   float qf[HPW][VEC];
 #pragma unroll
@@ -243,27 +315,39 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
   auto run = [&](auto hint_c) {
     constexpr bool kHint = decltype(hint_c)::value;
     for (int split = split0; split < P.nsplit; split += step) {
-      const int b0 = P.first + split * P.bps;
-      const int b1 = min(b0 + P.bps, P.first + P.pages);
-      const int tb = max(P.start, b0 * a.block_size);
-      const int te = min(n, b1 * a.block_size);
-
+      const int s0 = P.first + split * P.bps;
+      const int s1 = min(s0 + P.bps, P.first + P.pages);
+      const int parts = ceil_div(s1 - s0, P.pps);
       float m[HPW], l[HPW];
       float acc[HPW][VEC];
+      auto reset = [&]() {
 #pragma unroll
-      for (int h = 0; h < HPW; ++h) {
-        m[h] = -INFINITY;
-        l[h] = 0.f;
+        for (int h = 0; h < HPW; ++h) {
+          m[h] = -INFINITY;
+          l[h] = 0.f;
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) acc[h][i] = 0.f;
-      }
+          for (int i = 0; i < VEC; ++i) acc[h][i] = 0.f;
+        }
+      };
+      reset();
+      // This wave's pages: all parts of the split, or its own one. The table is
+      // read 64 pages at a time at most, whole parts where they fit, so chunks
+      // start at the same tokens either way.
+      const int b0 = WAVES > 1 ? min(s0 + wave * P.pps, s1) : s0;
+      const int b1 = WAVES > 1 ? min(b0 + P.pps, s1) : s1;
+      const int tb = max(P.start, b0 * a.block_size);
+      const int te = min(n, b1 * a.block_size);
+      const int seg_pages = P.pps <= 64 ? 64 / P.pps * P.pps : 64;
+      int pe = (b0 + P.pps) * a.block_size;  // end of the current part (token)
+      int folded = 0;
 
-      for (int seg = b0; seg < b1; seg += 64) {
+      for (int seg = b0, seg1; seg < b1; seg = seg1) {
+        seg1 = min(b1, seg + seg_pages);
+        if (P.pps > 64) seg1 = min(seg1, pe / a.block_size);
         const bool in_seg = seg + lane < b1;
         const int tbl = in_seg ? table[seg + lane] : 0;
         const int s_tb = max(tb, seg * a.block_size);
-        const int s_te = min(te, (seg + 64) * a.block_size);
-        if (s_tb >= s_te) continue;
+        const int s_te = min(te, seg1 * a.block_size);
         // Pages this row shares with a neighbouring row of the batch (the same
         // block at the same table index: parallel samples of one prompt, batches
         // grouped by prefix) are read with ordinary loads, so that the rows'
@@ -278,11 +362,11 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
         }
         // Branch-free loads: positions past the end re-read the last valid token
         // (masked out of the softmax), so a chunk is one straight run of loads.
-        auto issue = [&](int p0, raw_t (&kr)[U], raw_t (&vr)[U], auto stream_c) {
+        auto issue = [&](int p0, int p1, raw_t (&kr)[U], raw_t (&vr)[U], auto stream_c) {
           constexpr bool kStream = decltype(stream_c)::value;
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            const int pos = min(p0 + u * TPL + tg, s_te - 1);
+            const int pos = min(p0 + u * TPL + tg, p1 - 1);
             int page, off;
             if (a.bs_shift >= 0) {
               page = pos >> a.bs_shift;
@@ -301,11 +385,11 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
             }
           }
         };
-        // The chunk at p0 is read with ordinary loads when one of its pages is
+        // The chunk [p0, p1) is read with ordinary loads when one of its pages is
         // shared with a neighbouring row (wave-uniform).
-        auto load_chunk = [&](int p0, raw_t (&kr)[U], raw_t (&vr)[U]) {
+        auto load_chunk = [&](int p0, int p1, raw_t (&kr)[U], raw_t (&vr)[U]) {
           if constexpr (kHint) {
-            const int last = min(p0 + CH, s_te) - 1;
+            const int last = p1 - 1;
             int lo, hi;
             if (a.bs_shift >= 0) {
               lo = (p0 >> a.bs_shift) - seg;
@@ -316,15 +400,17 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
             }
             const uint64_t span = hi - lo >= 63 ? ~0ull : ((2ull << (hi - lo)) - 1);
             if ((shared_pages >> lo) & span) {
-              issue(p0, kr, vr, std::false_type{});
+              issue(p0, p1, kr, vr, std::false_type{});
               return;
             }
           }
-          issue(p0, kr, vr, std::true_type{});
+          issue(p0, p1, kr, vr, std::true_type{});
         };
         raw_t kr[U], vr[U];
-        load_chunk(s_tb, kr, vr);
-        for (int p0 = s_tb; p0 < s_te; p0 += CH) {
+        int lim = WAVES == 1 ? min(s_te, pe) : s_te;  // chunks end at the part's end
+        int p1 = min(s_tb + CH, lim);
+        load_chunk(s_tb, p1, kr, vr);
+        for (int p0 = s_tb; p0 < s_te;) {
           float sc[HPW][U];
           float mx[HPW];
 #pragma unroll
@@ -333,16 +419,14 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
           for (int u = 0; u < U; ++u) {
             float kf[VEC];
             if constexpr (!kDot2) unpack<T, VEC>(kr[u], kf);
-            const bool visible = p0 + u * TPL + tg < s_te;
+            const bool visible = p0 + u * TPL + tg < p1;
 #pragma unroll
             for (int h = 0; h < HPW; ++h) {
               float d = 0.f;
               if constexpr (kDot2) {
 #pragma unroll
                 for (int i = 0; i < VEC / 2; ++i)
-                  d = __builtin_amdgcn_fdot2_f32_bf16(
-                      __builtin_bit_cast(bf16x2_t, qp2[h][i]),
-                      __builtin_bit_cast(bf16x2_t, (uint32_t)kr[u][i]), d, false);
+                  d = dot2<T>(qp2[h][i], (uint32_t)kr[u][i], d);
                 d = group_sum<LPT>(d) * a.scale_log2;
               } else {
 #pragma unroll
@@ -376,8 +460,39 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
           }
 #pragma unroll
           for (int h = 0; h < HPW; ++h) m[h] = mx[h];
-          if (p0 + CH < s_te) load_chunk(p0 + CH, kr, vr);
+          p0 = p1;
+          bool part_end = false;
+          if (WAVES == 1 && p0 == lim) {
+            part_end = p0 == pe && p0 < te;
+            if (part_end) pe += P.pps * a.block_size;
+            lim = min(s_te, pe);
+          }
+          // Parts are folded in order: by the one wave through its LDS slot, or,
+          // in a workgroup of several waves, by wave 0 below.
+          auto end_part = [&]() {
+            if (folded > 0) fold_state<HPW, VEC>(lds, lane, m, l, acc, true);
+            store_state<HPW, VEC>(lds, lane, m, l, acc);
+            reset();
+            ++folded;
+          };
+          // One head: the next chunk's loads go out before the fold. Several:
+          // their registers are not free until after it.
+          if (WAVES == 1 && HPW > 1 && part_end) end_part();
+          if (p0 < s_te) {
+            p1 = min(p0 + CH, lim);
+            load_chunk(p0, p1, kr, vr);
+          }
+          if (WAVES == 1 && HPW == 1 && part_end) end_part();
         }
+      }
+      if (WAVES == 1 && folded > 0) fold_state<HPW, VEC>(lds, lane, m, l, acc, true);
+      if constexpr (WAVES > 1) {
+        constexpr int kSlot = HPW * (VEC + 2) * 64;
+        if (wave > 0 && wave < parts) store_state<HPW, VEC>(lds + (wave - 1) * kSlot, lane, m, l, acc);
+        __syncthreads();
+        if (wave > 0) return;
+        for (int w = 1; w < parts; ++w)
+          fold_state<HPW, VEC>(lds + (w - 1) * kSlot, lane, m, l, acc, false);
       }
 
 #pragma unroll
@@ -469,13 +584,23 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
   return true;
 }
 
+// Splits of a launch up to which each split gets a workgroup, one wave a part:
+// with more, single waves fill the chip by themselves. VALU kernel: 2 rows of
+// 24000 tokens (512 splits) 74 against 95 us, 4 rows of 4000 (1024) 34 against
+// 30. MFMA kernel (8 kv heads): 6 rows of 24000 (768) 128 against 140, 8 rows of
+// 4000-8000 (1024) 55 against 58.
+constexpr int kWideSplits = 512;
+constexpr int kWideMfmaSplits = 1024;
+
 // Grid form: one wave per (split column, group of HPW q heads, row).
-template <typename T, int VEC, int LPT, int HPW>
-__global__ __launch_bounds__(64) void paged_decode_kernel(DecodeArgs a) {
+template <typename T, int VEC, int LPT, int HPW, int WAVES>
+__global__ __launch_bounds__(WAVES > 1 ? 64 * WAVES : 64) void paged_decode_kernel(DecodeArgs a) {
+  constexpr int kSlots = WAVES > 1 ? WAVES - 1 : WAVES;
+  __shared__ float state[kSlots > 0 ? kSlots * HPW * (VEC + 2) * 64 : 1];
   int64_t row;
   int split0;
   if (!grid_slot(a, row, split0)) return;
-  decode_work<T, VEC, LPT, HPW>(a, row, (int)blockIdx.y * HPW, split0, gridDim.x);
+  decode_work<T, VEC, LPT, HPW, WAVES>(a, row, (int)blockIdx.y * HPW, split0, gridDim.x, state);
 }
 
 // ------------------------------------------------ grouped-query heads on MFMA
@@ -543,15 +668,48 @@ __device__ __forceinline__ u32x2_t lds_tr16(const uint16_t* p) {
   return __builtin_bit_cast(u32x2_t, r);
 }
 
-template <typename T, int D>
+// A wave's state in LDS: the group's columns of each accumulator register.
+template <int DT>
+__device__ __forceinline__ void store_state(float* p, int step, float m, float l,
+                                            const f32x4_t (&acc)[DT]) {
+  p[0] = m;
+  p[step] = l;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[(2 + 4 * t + i) * step] = acc[t][i];
+}
+
+// Combines the state in LDS with the one in registers, as fold_state above
+// (the reference maxima are finite here).
+template <int DT>
+__device__ __forceinline__ void fold_state(const float* p, int step, float& m, float& l,
+                                           f32x4_t (&acc)[DT], bool lds_first) {
+  const float mo = p[0], lo = p[step];
+  const float top = fmaxf(m, mo);
+  const float wr = fast_exp2(m - top), wo = fast_exp2(mo - top);
+  const float w0 = lds_first ? wo : wr, w1 = lds_first ? wr : wo;
+  m = top;
+  l = fmaf(lds_first ? l : lo, w1, (lds_first ? lo : l) * w0);
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float o = p[(2 + 4 * t + i) * step];
+      acc[t][i] = fmaf(lds_first ? acc[t][i] : o, w1, (lds_first ? o : acc[t][i]) * w0);
+    }
+}
+
+template <typename T, int D, int WAVES>
 __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t row, int head0,
-                                                 int split0, int step, uint16_t* vt) {
+                                                 int split0, int step, uint16_t* vt, float* lds) {
   constexpr int DC = D / 32;           // 32-dim k chunks of S = K Q^T
   constexpr int DT = D / 16;           // 16-dim tiles of O^T
   constexpr int KCH = D / 8;           // 16-byte chunks per token row
   constexpr int RPI = 64 / KCH;        // token rows per V staging instruction
   constexpr int NV = kMfmaChunk / RPI; // V staging loads per chunk
   const int lane = threadIdx.x & 63;
+  const int wave = WAVES > 1 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int col = lane & 15;
   const int grp = lane >> 4;
   const int kvh = head0 / a.group;
@@ -562,7 +720,7 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
   T* out = reinterpret_cast<T*>(a.out) + qrow * a.o_row + (int64_t)(head0 + col) * a.o_head +
            4 * grp;
   if (n == 0) {
-    if (split0 == 0 && hcol) {
+    if (split0 == 0 && wave == 0 && hcol) {
 #pragma unroll
       for (int t = 0; t < DT; ++t) *reinterpret_cast<u32x2_t*>(out + 16 * t) = u32x2_t{0u, 0u};
     }
@@ -621,21 +779,34 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
   };
 
   for (int split = split0; split < P.nsplit; split += step) {
-    const int b0 = P.first + split * P.bps;
-    const int b1 = min(b0 + P.bps, P.first + P.pages);
+    // Parts of the split as in decode_work: all of them, or this wave's one.
+    const int s0 = P.first + split * P.bps;
+    const int s1 = min(s0 + P.bps, P.first + P.pages);
+    const int b0 = WAVES > 1 ? min(s0 + wave * P.pps, s1) : s0;
+    const int b1 = WAVES > 1 ? min(b0 + P.pps, s1) : s1;
     const int tb = max(P.start, b0 * a.block_size);
     const int te = min(n, b1 * a.block_size);
+    const int seg_pages = P.pps <= 64 ? 64 / P.pps * P.pps : 64;
+    const int state_step = 4 * a.group;
+    const int state_size = (2 + 4 * DT) * state_step;
+    float* state = lds + grp * a.group + col;
+    int pe_page = b0 + P.pps;  // end of the current part
+    int folded = 0;
     float m = -1e30f;  // reference max (log2 domain) of this lane's head column
     float lsum = 0.f;  // partial sum over this lane's token slots
     f32x4_t acc[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    for (int seg = b0; seg < b1; seg += 64) {
+    for (int seg = b0, seg1; seg < b1; seg = seg1) {
+      seg1 = min(b1, seg + seg_pages);
+      if (P.pps > 64) seg1 = min(seg1, pe_page);
       const int tbl = (seg + lane < b1) ? table[seg + lane] : 0;
       const int s_tb = max(tb, seg * a.block_size);
-      const int s_te = min(te, (seg + 64) * a.block_size);
-      for (int p0 = s_tb; p0 < s_te; p0 += kMfmaChunk) {
+      const int s_te = min(te, seg1 * a.block_size);
+      for (int p0 = s_tb, p1; p0 < s_te; p0 = p1) {
+        // Chunks end at the part's end.
+        p1 = min(min(p0 + kMfmaChunk, s_te), pe_page * a.block_size);
         // Loads (branch-free: positions past the end re-read the last token).
         // The A-operand layout gives each token 4 lanes (64 bytes) per
         // instruction, so instructions c and c + 1 read the two halves of one
@@ -644,7 +815,7 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
         u32x4_t kop[2][DC];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          const int pos = min(p0 + 16 * t + col, s_te - 1);
+          const int pos = min(p0 + 16 * t + col, p1 - 1);
           const T* kp = kbase + page_addr(pos, tbl, seg, a.k_block, a.k_token);
 #pragma unroll
           for (int c = 0; c < DC; ++c) kop[t][c] = *reinterpret_cast<const u32x4_t*>(kp + 32 * c);
@@ -653,7 +824,7 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
         // have returned (its PV MFMAs consumed them), so the tile is free.
 #pragma unroll
         for (int r = 0; r < NV; ++r) {
-          const int pos = min(p0 + v_row + RPI * r, s_te - 1);
+          const int pos = min(p0 + v_row + RPI * r, p1 - 1);
           const T* vp = vbase[r % SWP] + page_addr(pos, tbl, seg, a.v_block, a.v_token);
           lds_dma16(vp, __builtin_amdgcn_readfirstlane(vt_lds + 1024 * r));
         }
@@ -665,7 +836,7 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
 #pragma unroll
           for (int c = 0; c < DC; ++c) sc[t] = Mfma16<T>::run(kop[t][c], qop[c], sc[t]);
         }
-        const int lim = s_te - p0 - 4 * grp;  // token slot t*16 + i visible when < lim
+        const int lim = p1 - p0 - 4 * grp;  // token slot t*16 + i visible when < lim
         float mx = -INFINITY;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -702,7 +873,29 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
           const u32x2_t hi = lds_tr16(vt + tr_off[t] + 16 * D);
           acc[t] = Mfma16<T>::run(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pop, acc[t]);
         }
+        if (WAVES == 1 && p1 == pe_page * a.block_size && p1 < te) {
+          pe_page += P.pps;
+          if (hcol) {
+            if (folded > 0) fold_state<DT>(state, state_step, m, lsum, acc, true);
+            store_state<DT>(state, state_step, m, lsum, acc);
+          }
+          m = -1e30f;
+          lsum = 0.f;
+#pragma unroll
+          for (int t = 0; t < DT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          ++folded;
+        }
       }
+    }
+    if (folded > 0 && hcol) fold_state<DT>(state, state_step, m, lsum, acc, true);
+    if constexpr (WAVES > 1) {
+      const int parts = ceil_div(s1 - s0, P.pps);
+      if (wave > 0 && wave < parts && hcol)
+        store_state<DT>(state + (wave - 1) * state_size, state_step, m, lsum, acc);
+      __syncthreads();
+      if (wave > 0) return;
+      for (int w = 1; w < parts; ++w)
+        if (hcol) fold_state<DT>(state + (w - 1) * state_size, state_step, m, lsum, acc, false);
     }
     const float L = lsum + shfl_xor_f32(lsum, 16);
     const float L4 = L + shfl_xor_f32(L, 32);
@@ -728,13 +921,31 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
   }
 }
 
-template <typename T, int D>
-__global__ __launch_bounds__(64) void paged_decode_mfma_kernel(DecodeArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t vt[kMfmaChunk * D];
+// Dynamic LDS: mfma_state_bytes per state (one, or WAVES - 1).
+template <typename T, int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 ? 3 : 2)))
+void paged_decode_mfma_kernel(DecodeArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t vt[WAVES][kMfmaChunk * D];
+  extern __shared__ float mfma_state[];
   int64_t row;
   int split0;
   if (!grid_slot(a, row, split0)) return;
-  decode_work_mfma<T, D>(a, row, (int)blockIdx.y * a.group, split0, gridDim.x, vt);
+  decode_work_mfma<T, D, WAVES>(a, row, (int)blockIdx.y * a.group, split0, gridDim.x,
+                                vt[WAVES > 1 ? threadIdx.x >> 6 : 0], mfma_state);
+}
+
+inline size_t mfma_state_bytes(int head_dim, int group) {
+  return (size_t)(2 + head_dim / 4) * 4 * group * sizeof(float);
+}
+
+// `waves` as in decode_work.
+template <typename T, int D>
+void launch_mfma(int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
+  const size_t state = mfma_state_bytes(D, a.group);
+  if (waves > 1)
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<T, D, 4>), grid, dim3(256), 3 * state, s, a);
+  else
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<T, D, 1>), grid, dim3(64), waves > 0 ? state : 0, s, a);
 }
 
 // Log-sum-exp merge of one (row, q head)'s split partials by one wave, for
@@ -807,32 +1018,48 @@ void launch_merge(int head_dim, dim3 grid, hipStream_t s, const DecodeArgs& a) {
   }
 }
 
+template <typename T, int VEC, int LPT, int HPW>
+void launch_waves(int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
+  if (waves == 8)
+    hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 8>), grid, dim3(512), 0, s, a);
+  else if (waves == 4)
+    hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 4>), grid, dim3(256), 0, s, a);
+  else if (waves == 1)
+    hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 1>), grid, dim3(64), 0, s, a);
+  else
+    hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 0>), grid, dim3(64), 0, s, a);
+}
+
 template <typename T, int VEC, int LPT>
-bool launch_hpw(int hpw, dim3 grid, hipStream_t s, const DecodeArgs& a) {
+bool launch_hpw(int hpw, int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
   switch (hpw) {
-    case 1: hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, 1>), grid, dim3(64), 0, s, a); return true;
-    case 2: hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, 2>), grid, dim3(64), 0, s, a); return true;
-    case 4: hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, 4>), grid, dim3(64), 0, s, a); return true;
-    case 8: hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, 8>), grid, dim3(64), 0, s, a); return true;
+    case 1: launch_waves<T, VEC, LPT, 1>(waves, grid, s, a); return true;
+    case 2: launch_waves<T, VEC, LPT, 2>(waves, grid, s, a); return true;
+    case 4: launch_waves<T, VEC, LPT, 4>(waves, grid, s, a); return true;
+    case 8: launch_waves<T, VEC, LPT, 8>(waves, grid, s, a); return true;
     default: return false;
   }
 }
 
 // Instantiations: every (VEC, LPT) for one head per wave; grouped heads per
 // wave (HPW > 1) only for full-width lanes of the usual head dims
-// (16-byte vectors, LPT 4, 8 or 16: head_dim 32, 64, 128 in 16-bit types).
+// (16-byte vectors, LPT 4 to 32: head_dim 32, 64, 128); parts (WAVES > 0)
+// likewise.
 template <typename T, int VEC>
-bool launch_vec(int lpt, int hpw, dim3 grid, hipStream_t s, const DecodeArgs& a) {
+bool launch_vec(int lpt, int hpw, int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
   constexpr bool kWide = VEC * (int)sizeof(T) == 16;
   switch (lpt) {
 #define VRH_LPT(L)                                                                 \
   case L:                                                                          \
-    if (hpw == 1) {                                                                \
-      hipLaunchKernelGGL((paged_decode_kernel<T, VEC, L, 1>), grid, dim3(64), 0, s, a); \
+    if constexpr (kWide && L >= 4 && L <= 16) return launch_hpw<T, VEC, L>(hpw, waves, grid, s, a); \
+    if (hpw != 1) return false;                                                    \
+    if constexpr (kWide && L == 32) {                                              \
+      launch_waves<T, VEC, L, 1>(waves, grid, s, a);                                \
       return true;                                                                 \
     }                                                                              \
-    if constexpr (kWide && L >= 4 && L <= 16) return launch_hpw<T, VEC, L>(hpw, grid, s, a); \
-    return false;
+    if (waves != 0) return false;                                                        \
+    hipLaunchKernelGGL((paged_decode_kernel<T, VEC, L, 1, 0>), grid, dim3(64), 0, s, a); \
+    return true;
     VRH_LPT(1)
     VRH_LPT(2)
     VRH_LPT(4)
@@ -846,13 +1073,13 @@ bool launch_vec(int lpt, int hpw, dim3 grid, hipStream_t s, const DecodeArgs& a)
 }
 
 template <typename T>
-bool launch_decode(int vec, int lpt, int hpw, dim3 grid, hipStream_t s, const DecodeArgs& a) {
+bool launch_decode(int vec, int lpt, int hpw, int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
   switch (vec) {
-    case 1: return launch_vec<T, 1>(lpt, hpw, grid, s, a);
-    case 2: return launch_vec<T, 2>(lpt, hpw, grid, s, a);
-    case 4: return launch_vec<T, 4>(lpt, hpw, grid, s, a);
+    case 1: return launch_vec<T, 1>(lpt, hpw, waves, grid, s, a);
+    case 2: return launch_vec<T, 2>(lpt, hpw, waves, grid, s, a);
+    case 4: return launch_vec<T, 4>(lpt, hpw, waves, grid, s, a);
     case 8:
-      if constexpr (sizeof(T) == 2) return launch_vec<T, 8>(lpt, hpw, grid, s, a);
+      if constexpr (sizeof(T) == 2) return launch_vec<T, 8>(lpt, hpw, waves, grid, s, a);
       return false;
     default: return false;
   }
@@ -964,8 +1191,14 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)head_dim));
   // Pages per split: at least kSplitTokens tokens; without a workspace every
   // row is a single split (pages can never exceed the table width).
-  a.min_bps = workspace != nullptr ? std::max(1, kSplitTokens / block_size)
+  const int split_tokens = std::min(kSplitTokens, kSplitBytes / (head_dim * es));
+  a.min_bps = workspace != nullptr ? std::max(1, split_tokens / block_size)
                                    : std::max(1, table_width);
+
+  // Rows too long for the shortest splits: at least twice as many tokens (up to
+  // kSplitTokens), so that rows of like length, which share prefix pages, keep
+  // splits that start at the same tokens.
+  a.long_bps = std::max(a.min_bps, std::min(kSplitTokens, 2 * split_tokens) / block_size);
 
   // Grouped-query heads per wave: the largest of 8, 4, 2 dividing the group
   // (1 without grouping, or where no grouped instantiation exists).
@@ -984,6 +1217,10 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   const bool mfma_gqa = (dtype == VRH_DTYPE_BF16 || dtype == VRH_DTYPE_F16) && vec * es == 16 &&
                         (head_dim == 64 || head_dim == 128) && a.group >= kMfmaMinGroup &&
                         a.group <= kMfmaHeads && (a.group >= kMfmaAllGroups || hpw < a.group);
+  // Other lane layouts have no workgroups of several waves, so no parts either.
+  const bool has_parts = vec * es == 16 && lpt >= 4 && lpt <= 32;
+  a.min_part = has_parts ? 2 * a.min_bps : 1 << 30;
+  a.max_parts = mfma_gqa ? kMfmaParts : kParts;
   // Largest split count any row of this table width can need: the grid is a
   // function of shapes only (graph capture), never of device lengths.
   const int max_pages = std::max(1, table_width);
@@ -995,22 +1232,31 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
     a.row_base = first;
     const unsigned count = (unsigned)std::min<int64_t>(rows - first, kRowsPerLaunch);
     bool ok = false;
+    // Splits of rows this table (and window) could hold: how many parts they can
+    // have, and whether each gets a workgroup (kWideSplits).
+    const int seen_pages =
+        window > 0 ? (int)std::min<int64_t>(max_pages, (int64_t)window / block_size + 2) : max_pages;
+    const int parts =
+        std::min(a.max_parts, ceil_div(std::max(a.long_bps, ceil_div(seen_pages, kMaxSplits)), a.min_part));
+    const int units = mfma_gqa ? kv_heads : q_heads / hpw;
+    const bool wide =
+        parts > 1 && (int64_t)gx * units * count <= (mfma_gqa ? kWideMfmaSplits : kWideSplits);
+    const int waves = parts <= 1 ? 0 : !wide ? 1 : parts > 4 ? 8 : 4;
+    const dim3 grid((unsigned)gx, (unsigned)units, count);
     if (mfma_gqa) {
-      dim3 grid((unsigned)gx, (unsigned)kv_heads, count);
       ok = true;
       if (dtype == VRH_DTYPE_BF16) {
-        if (head_dim == 128) hipLaunchKernelGGL((paged_decode_mfma_kernel<bf16_t, 128>), grid, dim3(64), 0, s, a);
-        else hipLaunchKernelGGL((paged_decode_mfma_kernel<bf16_t, 64>), grid, dim3(64), 0, s, a);
+        if (head_dim == 128) launch_mfma<bf16_t, 128>(waves, grid, s, a);
+        else launch_mfma<bf16_t, 64>(waves, grid, s, a);
       } else {
-        if (head_dim == 128) hipLaunchKernelGGL((paged_decode_mfma_kernel<f16_t, 128>), grid, dim3(64), 0, s, a);
-        else hipLaunchKernelGGL((paged_decode_mfma_kernel<f16_t, 64>), grid, dim3(64), 0, s, a);
+        if (head_dim == 128) launch_mfma<f16_t, 128>(waves, grid, s, a);
+        else launch_mfma<f16_t, 64>(waves, grid, s, a);
       }
     } else {
-      dim3 grid((unsigned)gx, (unsigned)(q_heads / hpw), count);
       switch (dtype) {
-        case VRH_DTYPE_F32: ok = launch_decode<float>(vec, lpt, hpw, grid, s, a); break;
-        case VRH_DTYPE_F16: ok = launch_decode<f16_t>(vec, lpt, hpw, grid, s, a); break;
-        case VRH_DTYPE_BF16: ok = launch_decode<bf16_t>(vec, lpt, hpw, grid, s, a); break;
+        case VRH_DTYPE_F32: ok = launch_decode<float>(vec, lpt, hpw, waves, grid, s, a); break;
+        case VRH_DTYPE_F16: ok = launch_decode<f16_t>(vec, lpt, hpw, waves, grid, s, a); break;
+        case VRH_DTYPE_BF16: ok = launch_decode<bf16_t>(vec, lpt, hpw, waves, grid, s, a); break;
       }
     }
     VRH_CHECK_ARG(ok, "%s: no kernel for vec=%d lanes=%d heads/wave=%d", who, vec, lpt, hpw);

@@ -58,7 +58,7 @@ constexpr int kBM = kWQ * kWaves;          // queries per workgroup
 constexpr int kSB = 32;                    // keys per sub-block (one pipeline step)
 constexpr int kStages = 3;                 // LDS stages: one sub-block each
 constexpr int kTableSeg = 512;             // page ids staged in LDS at a time
-constexpr int kMinRun = 4;                 // sub-blocks of the shortest key split
+constexpr int kMinRun = 8;                 // sub-blocks of the shortest key split
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
