@@ -18,8 +18,12 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/library.h>
 
 #include "vllm_rlt_hip.h"
@@ -328,6 +332,128 @@ TORCH_LIBRARY_IMPL(vllm_rlt_hip, CUDA, ops) {
   ops.impl("kv_copy_blocks", &kv_copy_blocks);
 }
 
-// An empty Python module: importing it runs the registrations above.
-static PyModuleDef vrh_module = {PyModuleDef_HEAD_INIT, "_C", nullptr, -1, nullptr};
+// ------------------------------------------------ calls from the Python adapter
+// decode, prefill, append and silu of this module take exactly the plain calls
+// (ordinary ROCm tensors that pass every check of vllm_rlt/kernels) and answer
+// None to all others, which the adapter then handles, or refuses with its own
+// errors. They skip the adapter's per-call host work: 20.6 us a decode call
+// through Python and ctypes, 10.1 through the dispatcher's op (64 rows), which
+// is longer than the kernels of a small call.
+namespace {
+
+const at::Tensor* plain(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() ? &t : nullptr;
+}
+
+// The first n arguments as tensors of one device; false if one is not plain.
+bool plain_args(PyObject* const* args, int n, const at::Tensor** t) {
+  if (at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set())
+    return false;
+  for (int i = 0; i < n; ++i) {
+    t[i] = plain(args[i]);
+    if (t[i] == nullptr || t[i]->device() != t[0]->device()) return false;
+  }
+  return true;
+}
+
+bool known_dtype(const at::Tensor& t) {
+  const auto d = t.scalar_type();
+  return d == at::kFloat || d == at::kHalf || d == at::kBFloat16;
+}
+
+bool small_int(PyObject* o, int64_t* v) {
+  if (!PyLong_CheckExact(o)) return false;
+  int overflow = 0;
+  *v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow == 0 && *v >= 0 && *v < (1ll << 31);
+}
+
+// q, key cache, value cache, tables, lengths as check_attention wants them,
+// nothing to copy.
+bool plain_attention(const at::Tensor* const* t) {
+  const at::Tensor &q = *t[0], &kc = *t[1], &vc = *t[2], &tables = *t[3], &lengths = *t[4];
+  return q.dim() == 3 && known_dtype(q) && q.stride(2) == 1 && q.size(0) > 0 && q.size(1) > 0 &&
+         kc.dim() == 4 && kc.scalar_type() == q.scalar_type() &&
+         vc.scalar_type() == q.scalar_type() && vc.sizes() == kc.sizes() &&
+         kc.size(3) == q.size(2) && kc.stride(3) == 1 && vc.stride(3) == 1 && kc.size(2) > 0 &&
+         q.size(1) % kc.size(2) == 0 && tables.dim() == 2 && tables.scalar_type() == at::kInt &&
+         (tables.size(1) == 0 || tables.stride(1) == 1) && lengths.dim() == 1 &&
+         lengths.scalar_type() == at::kInt && lengths.is_contiguous() &&
+         lengths.size(0) == tables.size(0);
+}
+
+PyObject* none() { Py_RETURN_NONE; }
+
+PyObject* py_decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* t[5];
+  int64_t window;
+  if (n != 6 || !plain_args(args, 5, t) || !plain_attention(t) || !small_int(args[5], &window) ||
+      t[3]->size(0) != t[0]->size(0))
+    return none();
+  return THPVariable_Wrap(paged_attention(*t[0], *t[1], *t[2], *t[3], *t[4], window));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* t[6];
+  int64_t max_q;
+  if (n != 7 || !plain_args(args, 6, t) || !plain_attention(t) || !small_int(args[6], &max_q) ||
+      t[5]->dim() != 1 || t[5]->scalar_type() != at::kInt || !t[5]->is_contiguous() ||
+      t[3]->size(0) < 1 || t[5]->size(0) != t[3]->size(0) + 1)
+    return none();
+  return THPVariable_Wrap(paged_prefill(*t[0], *t[1], *t[2], *t[3], *t[4], *t[5], max_q));
+  END_HANDLE_TH_ERRORS
+}
+
+// key cache, value cache (layer views), k, v, write blocks, write offsets; no
+// mask, no active row count. True when done.
+PyObject* py_append(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* t[6];
+  if (n != 6 || !plain_args(args, 6, t)) return none();
+  const at::Tensor &kc = *t[0], &vc = *t[1], &blocks = *t[4], &offsets = *t[5];
+  if (kc.dim() != 4 || !known_dtype(kc) || vc.scalar_type() != kc.scalar_type() ||
+      vc.sizes() != kc.sizes() || vc.strides() != kc.strides() || kc.stride(3) != 1)
+    return none();
+  for (const at::Tensor* x : {t[2], t[3]})
+    if (x->dim() != 3 || x->scalar_type() != kc.scalar_type() || x->size(1) != kc.size(2) ||
+        x->size(2) != kc.size(3) || x->stride(2) != 1)
+      return none();
+  const int64_t rows = t[2]->size(0);
+  if (rows == 0 || t[3]->size(0) != rows) return none();
+  for (const at::Tensor* x : {&blocks, &offsets})
+    if (x->dim() != 1 || x->scalar_type() != at::kLong || x->size(0) < rows || !x->is_contiguous())
+      return none();
+  kv_append(kc, vc, *t[2], *t[3], blocks, offsets, std::nullopt, std::nullopt);
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* t[2];
+  if (n != 2 || !plain_args(args, 2, t) || !known_dtype(*t[0]) ||
+      t[0]->scalar_type() != t[1]->scalar_type() || t[0]->sizes() != t[1]->sizes() ||
+      !t[0]->is_contiguous() || !t[1]->is_contiguous() ||
+      (at::GradMode::is_enabled() && (t[0]->requires_grad() || t[1]->requires_grad())))
+    return none();
+  return THPVariable_Wrap(silu_and_mul(*t[0], *t[1]));
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef vrh_methods[] = {
+    {"decode", (PyCFunction)(void (*)(void))py_decode, METH_FASTCALL, nullptr},
+    {"prefill", (PyCFunction)(void (*)(void))py_prefill, METH_FASTCALL, nullptr},
+    {"append", (PyCFunction)(void (*)(void))py_append, METH_FASTCALL, nullptr},
+    {"silu", (PyCFunction)(void (*)(void))py_silu, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+}  // namespace
+
+// Importing the module runs the registrations above.
+static PyModuleDef vrh_module = {PyModuleDef_HEAD_INIT, "_C", nullptr, -1, vrh_methods};
 PyMODINIT_FUNC PyInit__C(void) { return PyModule_Create(&vrh_module); }

@@ -29,3 +29,11 @@ def load_extension() -> None:
     if not try_load_extension():
         raise RuntimeError(
             "The torch operator library vllm_rlt._C is not built: run make in vllm-rlt_amd.")
+
+
+@cache
+def plain_calls():
+    """The module's ``decode``/``prefill``/``append``/``silu`` (see torch_ops.cpp), which
+    take plain calls of the adapter in one step and answer None to all others;
+    None where the module is not built."""
+    return import_module("vllm_rlt._C") if try_load_extension() else None

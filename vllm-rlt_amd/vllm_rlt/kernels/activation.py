@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import torch
 
+from vllm_rlt.kernels._extension import plain_calls
 from vllm_rlt.kernels._hip import VRH_DTYPE_BF16, VRH_DTYPE_F16, VRH_DTYPE_F32, library
 
 _CODES = {torch.float32: VRH_DTYPE_F32, torch.float16: VRH_DTYPE_F16,
@@ -40,6 +41,11 @@ def _validate_inputs(gate: torch.Tensor, up: torch.Tensor) -> None:
 
 def silu_and_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``F.silu(gate) * up`` with the SiLU rounded to the dtype, on the gfx950 kernel."""
+    plain = plain_calls()
+    if plain is not None:
+        out = plain.silu(gate, up)
+        if out is not None:
+            return out
     _validate_inputs(gate, up)
     if gate.device.type != "cuda":
         raise ValueError("silu_and_mul of the hip build needs ROCm device tensors")

@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import torch
 
+from vllm_rlt.kernels._extension import plain_calls
 from vllm_rlt.kernels._hip import VRH_DTYPE_BF16, VRH_DTYPE_F16, VRH_DTYPE_F32, library
 
 _DTYPE_CODES = {
@@ -98,6 +99,11 @@ def paged_attention(q, key_cache, value_cache, block_tables, context_lengths, wi
     """Single-query paged attention; ``window`` > 0 keeps the last ``window`` keys."""
     if type(window) is not int or window < 0:
         raise ValueError("window must be a nonnegative integer")
+    plain = plain_calls()
+    if plain is not None:
+        output = plain.decode(q, key_cache, value_cache, block_tables, context_lengths, window)
+        if output is not None:
+            return output
     q, context_lengths = _attention_inputs(q, key_cache, value_cache, block_tables,
                                            context_lengths)
     rows = q.shape[0]
@@ -161,6 +167,12 @@ def paged_attention_noalloc(q, key_cache, value_cache, block_tables, context_len
 def paged_prefill_attention(q, key_cache, value_cache, block_tables, context_lengths,
                             cu_seqlens_q, max_seqlen_q):
     """Packed causal prefill, bottom-right aligned per sequence."""
+    plain = plain_calls()
+    if plain is not None:
+        output = plain.prefill(q, key_cache, value_cache, block_tables, context_lengths,
+                               cu_seqlens_q, max_seqlen_q)
+        if output is not None:
+            return output
     q, context_lengths = _attention_inputs(q, key_cache, value_cache, block_tables,
                                            context_lengths)
     _check_int("cu_seqlens_q", cu_seqlens_q, torch.int32, 1, q.device)
@@ -225,6 +237,11 @@ def kv_append(key_cache, value_cache, k, v, write_blocks, write_offsets, *, writ
     ``[write_blocks[r], write_offsets[r]]`` unless ``write_mask[r]`` is false or
     ``r >= active_rows`` (a device int32 scalar). Bit-exact.
     """
+    if write_mask is None and active_rows is None:
+        plain = plain_calls()
+        if plain is not None and plain.append(key_cache, value_cache, k, v, write_blocks,
+                                              write_offsets):
+            return
     if key_cache.ndim != 4 or value_cache.shape != key_cache.shape:
         raise ValueError("caches must be matching [blocks, block_size, kv_heads, head_dim] views")
     if key_cache.stride() != value_cache.stride():
