@@ -186,8 +186,8 @@ size_t vrh_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t max_seqlen_q,
  * tile's keys into up to 16 runs computed side by side and merges their fp32
  * partials. A call given at least this many bytes does so; with fewer, down to
  * vrh_paged_prefill_workspace_bytes, it runs one workgroup per tile. The number
- * of runs follows from the call's shapes, so a query's last bits may differ
- * between calls of different shapes. */
+ * of runs follows from the call's shapes and lengths, so a query's last bits
+ * may differ between batches. */
 size_t vrh_paged_prefill_split_workspace_bytes(int64_t num_seqs, int64_t total_q,
                                                int32_t max_seqlen_q, int32_t q_heads,
                                                int32_t kv_heads, int32_t head_dim,
