@@ -93,3 +93,17 @@ def test_split_prefill_in_a_graph_follows_the_device_lengths(gpu):
         torch.cuda.synchronize()
         assert torch.equal(captured, paged_prefill_attention(q, k, v, tables, lengths, cu, max_q))
         assert_close(captured, oracle_prefill(q, k, v, tables, lengths, cu), torch.bfloat16)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(2, 2), (8, 2), (16, 8)])
+def test_longest_query_count_is_only_a_bound(gpu, heads, kv_heads):
+    """max_seqlen_q up to INT32_MAX is accepted, whatever the group, and changes
+    nothing: no sequence has more queries than the packed batch."""
+    from vllm_rlt.kernels.hip_attention import paged_prefill_attention
+
+    q, k, v, tables, lengths, cu, max_q = prefill_inputs([(300, 40), (77, 9)], heads, kv_heads, 64,
+                                                         torch.bfloat16, gpu, seed=2)
+    expected = paged_prefill_attention(q, k, v, tables, lengths, cu, max_q)
+    assert_close(expected, oracle_prefill(q, k, v, tables, lengths, cu), torch.bfloat16)
+    for bound in (q.shape[0], 2**31 - 1):
+        assert torch.equal(paged_prefill_attention(q, k, v, tables, lengths, cu, bound), expected)

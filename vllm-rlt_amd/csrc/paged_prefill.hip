@@ -1033,8 +1033,10 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
   a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)head_dim));
   a.num_seqs = num_seqs;
   a.kv_heads = kv_heads;
-  const int64_t qblocks = ceil_div64((int64_t)max_seqlen_q * a.group, kBM);
-  VRH_CHECK_ARG(qblocks < (1 << 24), "vrh_paged_prefill: too many work items");
+  // No sequence has more than total_q queries, so a max_seqlen_q that only bounds
+  // them from above (up to INT32_MAX) costs no tiles and is not refused.
+  const int64_t qblocks = ceil_div64(std::min<int64_t>(max_seqlen_q, total_q) * a.group, kBM);
+  VRH_CHECK_ARG(qblocks <= (1 << 24), "vrh_paged_prefill: too many work items");
   a.qblocks = (int32_t)qblocks;
   // Up to 64 sequences are ranked inside the kernel (also without a
   // workspace); larger batches use the ordering kernel and the workspace.
