@@ -900,6 +900,9 @@ constexpr int kMaxKeySplits = 16;
 // chunk (64 tiles) 18.1 against 19.5 us.
 constexpr int kMinSaved = 12;
 
+// Head dims of the MFMA tiles (16-bit types, 16-byte aligned rows).
+bool tile_head_dim(int32_t head_dim) { return head_dim >= 32 && head_dim <= 128 && head_dim % 32 == 0; }
+
 // Upper bound of the tiles per kv head of a batch whose sequences' query counts
 // sum to at most total_q, each at most max_seqlen_q.
 int64_t most_tiles(int64_t num_seqs, int64_t total_q, int32_t max_seqlen_q, int64_t group) {
@@ -912,7 +915,7 @@ int64_t most_tiles(int64_t num_seqs, int64_t total_q, int32_t max_seqlen_q, int6
 int32_t most_splits(int64_t num_seqs, int64_t total_q, int32_t max_seqlen_q, int32_t q_heads,
                     int32_t kv_heads, int32_t head_dim, int32_t block_size, int32_t table_width) {
   if (num_seqs < 1 || num_seqs > 64 || total_q < 1 || max_seqlen_q <= kExactQ || kv_heads < 1 ||
-      block_size < 1)
+      q_heads < kv_heads || block_size < 1 || !tile_head_dim(head_dim))
     return 1;
   const int64_t group = q_heads / kv_heads;
   const int64_t most = most_tiles(num_seqs, total_q, max_seqlen_q, group) * kv_heads;
@@ -965,7 +968,7 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
                 "vrh_paged_prefill: null pointer");
   hipStream_t s = (hipStream_t)stream;
   const bool half = dtype == VRH_DTYPE_BF16 || dtype == VRH_DTYPE_F16;
-  bool mfma = half && head_dim % 32 == 0 && head_dim <= 128 && block_size >= 1 &&
+  bool mfma = half && tile_head_dim(head_dim) && block_size >= 1 &&
               q_token_stride % 8 == 0 && q_head_stride % 8 == 0 && out_token_stride % 4 == 0 &&
               out_head_stride % 4 == 0 && k_block_stride % 8 == 0 && k_token_stride % 8 == 0 &&
               k_head_stride % 8 == 0 && v_block_stride % 8 == 0 && v_token_stride % 8 == 0 &&
