@@ -107,3 +107,25 @@ def test_longest_query_count_is_only_a_bound(gpu, heads, kv_heads):
     assert_close(expected, oracle_prefill(q, k, v, tables, lengths, cu), torch.bfloat16)
     for bound in (q.shape[0], 2**31 - 1):
         assert torch.equal(paged_prefill_attention(q, k, v, tables, lengths, cu, bound), expected)
+
+
+@pytest.mark.parametrize("dtype,offset,splits", [
+    (torch.bfloat16, 0, True), (torch.float32, 0, False), (torch.bfloat16, 1, False)])
+@pytest.mark.parametrize("plain", [True, False])
+def test_only_calls_on_tiles_hold_room_for_splits(gpu, dtype, offset, splits, plain, monkeypatch):
+    """A call that the tiles cannot take (float32, rows that are not 16-byte
+    aligned) allocates no partials, through the extension module or ctypes."""
+    from vllm_rlt.kernels import hip_attention
+
+    if not plain:
+        monkeypatch.setattr(hip_attention, "plain_calls", lambda: None)
+    q, k, v, tables, lengths, cu, max_q = prefill_inputs([(1500, 100)], 8, 8, 64, dtype, gpu)
+    shifted = torch.empty(q.numel() + offset, dtype=dtype, device=gpu)[offset:].view(q.shape)
+    q = shifted.copy_(q)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = hip_attention.paged_prefill_attention(q, k, v, tables, lengths, cu, max_q)
+    peak = torch.cuda.max_memory_allocated() - before
+    assert (peak > 1 << 20) == splits, peak  # the output and decode partials take 0.3 MiB
+    assert_close(out, oracle_prefill(q, k, v, tables, lengths, cu), dtype)

@@ -109,6 +109,17 @@ at::Tensor paged_attention(const at::Tensor& q_in, const at::Tensor& kc, const a
   return out;
 }
 
+// Prefill calls that can run on MFMA tiles (16-bit types, 16-byte aligned rows):
+// only these have a use for key-split partials.
+bool on_tiles(std::initializer_list<const at::Tensor*> tensors) {
+  for (const at::Tensor* t : tensors) {
+    if (t->element_size() != 2 || (uintptr_t)t->data_ptr() % 16 != 0) return false;
+    for (int64_t i = 0; i + 1 < t->dim(); ++i)
+      if (t->stride(i) % 8 != 0) return false;
+  }
+  return true;
+}
+
 at::Tensor paged_prefill(const at::Tensor& q_in, const at::Tensor& kc, const at::Tensor& vc,
                          const at::Tensor& tables, const at::Tensor& lengths_in,
                          const at::Tensor& cu_in, int64_t max_seqlen_q) {
@@ -125,9 +136,12 @@ at::Tensor paged_prefill(const at::Tensor& q_in, const at::Tensor& kc, const at:
   at::Tensor out = at::empty_like(q);
   if (q.size(0) == 0 || seqs == 0) return out;
   const int32_t heads = (int32_t)q.size(1), dim = (int32_t)q.size(2);
-  const size_t nbytes = vrh_paged_prefill_split_workspace_bytes(
-      seqs, q.size(0), (int32_t)max_seqlen_q, heads, (int32_t)kc.size(2), dim, (int32_t)kc.size(1),
-      (int32_t)tables.size(1));
+  const size_t nbytes =
+      on_tiles({&q, &kc, &vc})
+          ? vrh_paged_prefill_split_workspace_bytes(seqs, q.size(0), (int32_t)max_seqlen_q, heads,
+                                                    (int32_t)kc.size(2), dim, (int32_t)kc.size(1),
+                                                    (int32_t)tables.size(1))
+          : vrh_paged_prefill_workspace_bytes(seqs, (int32_t)max_seqlen_q, heads, dim);
   at::Tensor workspace = at::empty({(int64_t)nbytes}, q.options().dtype(at::kByte));
   check_rc(vrh_paged_prefill(dtype_code(q), out.data_ptr(), q.data_ptr(), kc.data_ptr(),
                              vc.data_ptr(), tables.data_ptr<int32_t>(),

@@ -164,6 +164,13 @@ def paged_attention_noalloc(q, key_cache, value_cache, block_tables, context_len
     return out
 
 
+def _on_tiles(*tensors):
+    """Prefill calls that can run on MFMA tiles (16-bit types, 16-byte aligned rows):
+    only these have a use for key-split partials."""
+    return all(t.element_size() == 2 and t.data_ptr() % 16 == 0
+               and all(stride % 8 == 0 for stride in t.stride()[:-1]) for t in tensors)
+
+
 def paged_prefill_attention(q, key_cache, value_cache, block_tables, context_lengths,
                             cu_seqlens_q, max_seqlen_q):
     """Packed causal prefill, bottom-right aligned per sequence."""
@@ -184,9 +191,12 @@ def paged_prefill_attention(q, key_cache, value_cache, block_tables, context_len
         return output
     cu_seqlens_q = cu_seqlens_q.contiguous()
     lib = library()
-    nbytes = lib.vrh_paged_prefill_split_workspace_bytes(
-        sequences, q.shape[0], int(max_seqlen_q), q.shape[1], key_cache.shape[2], q.shape[2],
-        key_cache.shape[1], block_tables.shape[1])
+    nbytes = lib.vrh_paged_prefill_workspace_bytes(sequences, int(max_seqlen_q), q.shape[1],
+                                                   q.shape[2])
+    if _on_tiles(q, key_cache, value_cache):
+        nbytes = lib.vrh_paged_prefill_split_workspace_bytes(
+            sequences, q.shape[0], int(max_seqlen_q), q.shape[1], key_cache.shape[2], q.shape[2],
+            key_cache.shape[1], block_tables.shape[1])
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
     lib.check(
         lib.vrh_paged_prefill(
