@@ -129,3 +129,34 @@ def test_only_calls_on_tiles_hold_room_for_splits(gpu, dtype, offset, splits, pl
     peak = torch.cuda.max_memory_allocated() - before
     assert (peak > 1 << 20) == splits, peak  # the output and decode partials take 0.3 MiB
     assert_close(out, oracle_prefill(q, k, v, tables, lengths, cu), dtype)
+
+
+@pytest.mark.parametrize("plain", [True, False])
+def test_call_without_room_for_splits_runs_unsplit(gpu, plain, monkeypatch):
+    """When the allocator cannot give the partials (a pool sized to the last of
+    the memory), the call runs as with the smaller workspace, bit for bit."""
+    from vllm_rlt.kernels import hip_attention
+    from vllm_rlt.kernels._hip import library
+
+    if not plain:
+        monkeypatch.setattr(hip_attention, "plain_calls", lambda: None)
+    inputs = prefill_inputs([(1500, 129)], 16, 16, 128, torch.bfloat16, gpu, seed=4)
+    base, full = sizes(library(), inputs)
+    assert full > base + (12 << 20)
+    unsplit = call(library(), inputs, base)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    held = []
+    try:
+        # Room for the output (0.5 MiB) and the small workspace (0.2 MiB) only.
+        torch.cuda.set_per_process_memory_fraction(
+            (torch.cuda.memory_reserved() + (8 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(12 << 20, dtype=torch.uint8, device=gpu))
+        out = hip_attention.paged_prefill_attention(*inputs)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        del held
+    assert torch.equal(out, unsplit)

@@ -136,13 +136,24 @@ at::Tensor paged_prefill(const at::Tensor& q_in, const at::Tensor& kc, const at:
   at::Tensor out = at::empty_like(q);
   if (q.size(0) == 0 || seqs == 0) return out;
   const int32_t heads = (int32_t)q.size(1), dim = (int32_t)q.size(2);
-  const size_t nbytes =
+  size_t nbytes = vrh_paged_prefill_workspace_bytes(seqs, (int32_t)max_seqlen_q, heads, dim);
+  const size_t wanted =
       on_tiles({&q, &kc, &vc})
           ? vrh_paged_prefill_split_workspace_bytes(seqs, q.size(0), (int32_t)max_seqlen_q, heads,
                                                     (int32_t)kc.size(2), dim, (int32_t)kc.size(1),
                                                     (int32_t)tables.size(1))
-          : vrh_paged_prefill_workspace_bytes(seqs, (int32_t)max_seqlen_q, heads, dim);
-  at::Tensor workspace = at::empty({(int64_t)nbytes}, q.options().dtype(at::kByte));
+          : nbytes;
+  at::Tensor workspace;
+  if (wanted > nbytes) {
+    // Without room for the partials the call still runs, unsplit.
+    try {
+      workspace = at::empty({(int64_t)wanted}, q.options().dtype(at::kByte));
+      nbytes = wanted;
+    } catch (const c10::OutOfMemoryError&) {
+    }
+  }
+  if (!workspace.defined())
+    workspace = at::empty({(int64_t)nbytes}, q.options().dtype(at::kByte));
   check_rc(vrh_paged_prefill(dtype_code(q), out.data_ptr(), q.data_ptr(), kc.data_ptr(),
                              vc.data_ptr(), tables.data_ptr<int32_t>(),
                              lengths.data_ptr<int32_t>(), cu.data_ptr<int32_t>(), seqs, q.size(0),

@@ -193,11 +193,20 @@ def paged_prefill_attention(q, key_cache, value_cache, block_tables, context_len
     lib = library()
     nbytes = lib.vrh_paged_prefill_workspace_bytes(sequences, int(max_seqlen_q), q.shape[1],
                                                    q.shape[2])
+    workspace = None
     if _on_tiles(q, key_cache, value_cache):
-        nbytes = lib.vrh_paged_prefill_split_workspace_bytes(
+        wanted = lib.vrh_paged_prefill_split_workspace_bytes(
             sequences, q.shape[0], int(max_seqlen_q), q.shape[1], key_cache.shape[2], q.shape[2],
             key_cache.shape[1], block_tables.shape[1])
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        if wanted > nbytes:
+            # Without room for the partials the call still runs, unsplit.
+            try:
+                workspace = torch.empty(wanted, dtype=torch.uint8, device=q.device)
+                nbytes = wanted
+            except torch.OutOfMemoryError:
+                pass
+    if workspace is None:
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
     lib.check(
         lib.vrh_paged_prefill(
             dtype_code(q.dtype), output.data_ptr(), q.data_ptr(), key_cache.data_ptr(),
