@@ -26,6 +26,9 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/library.h>
 
+#include <array>
+#include <initializer_list>
+
 #include "vllm_rlt_hip.h"
 
 namespace {
@@ -411,6 +414,22 @@ bool plain_attention(const at::Tensor* const* t) {
 
 PyObject* none() { Py_RETURN_NONE; }
 
+// f(tensors) without the interpreter lock, as the dispatcher's bindings and
+// ctypes call it: an allocation or a launch that has to wait (a full queue,
+// first use of a kernel) must not stop the other Python threads. The tensors
+// are handles of their own, since another thread may swap what an argument
+// holds; an exception takes the lock back on its way out.
+template <int N, typename F>
+auto unlocked(const at::Tensor* const* t, F f) {
+  std::array<at::Tensor, N> tensors;
+  for (int i = 0; i < N; ++i) tensors[i] = *t[i];
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return f(tensors);
+}
+
 PyObject* py_decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const at::Tensor* t[5];
@@ -418,7 +437,9 @@ PyObject* py_decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 6 || !plain_args(args, 5, t) || !plain_attention(t) || !small_int(args[5], &window) ||
       t[3]->size(0) != t[0]->size(0))
     return none();
-  return THPVariable_Wrap(paged_attention(*t[0], *t[1], *t[2], *t[3], *t[4], window));
+  return THPVariable_Wrap(unlocked<5>(t, [=](const auto& x) {
+    return paged_attention(x[0], x[1], x[2], x[3], x[4], window);
+  }));
   END_HANDLE_TH_ERRORS
 }
 
@@ -430,7 +451,9 @@ PyObject* py_prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
       t[5]->dim() != 1 || t[5]->scalar_type() != at::kInt || !t[5]->is_contiguous() ||
       t[3]->size(0) < 1 || t[5]->size(0) != t[3]->size(0) + 1)
     return none();
-  return THPVariable_Wrap(paged_prefill(*t[0], *t[1], *t[2], *t[3], *t[4], *t[5], max_q));
+  return THPVariable_Wrap(unlocked<6>(t, [=](const auto& x) {
+    return paged_prefill(x[0], x[1], x[2], x[3], x[4], x[5], max_q);
+  }));
   END_HANDLE_TH_ERRORS
 }
 
@@ -453,7 +476,9 @@ PyObject* py_append(PyObject*, PyObject* const* args, Py_ssize_t n) {
   for (const at::Tensor* x : {&blocks, &offsets})
     if (x->dim() != 1 || x->scalar_type() != at::kLong || x->size(0) < rows || !x->is_contiguous())
       return none();
-  kv_append(kc, vc, *t[2], *t[3], blocks, offsets, std::nullopt, std::nullopt);
+  unlocked<6>(t, [](const auto& x) {
+    kv_append(x[0], x[1], x[2], x[3], x[4], x[5], std::nullopt, std::nullopt);
+  });
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -466,7 +491,8 @@ PyObject* py_silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
       !t[0]->is_contiguous() || !t[1]->is_contiguous() ||
       (at::GradMode::is_enabled() && (t[0]->requires_grad() || t[1]->requires_grad())))
     return none();
-  return THPVariable_Wrap(silu_and_mul(*t[0], *t[1]));
+  return THPVariable_Wrap(
+      unlocked<2>(t, [](const auto& x) { return silu_and_mul(x[0], x[1]); }));
   END_HANDLE_TH_ERRORS
 }
 
