@@ -338,12 +338,14 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
       const int tb = max(P.start, b0 * a.block_size);
       const int te = min(n, b1 * a.block_size);
       const int seg_pages = P.pps <= 64 ? 64 / P.pps * P.pps : 64;
-      int pe = (b0 + P.pps) * a.block_size;  // end of the current part (token)
+      // End of the current part (page). Never past the wave's own pages: times
+      // block_size it has to stay in 32 bits for contexts close to 2^31 tokens.
+      int pe = min(b0 + P.pps, b1);
       int folded = 0;
 
       for (int seg = b0, seg1; seg < b1; seg = seg1) {
         seg1 = min(b1, seg + seg_pages);
-        if (P.pps > 64) seg1 = min(seg1, pe / a.block_size);
+        if (P.pps > 64) seg1 = min(seg1, pe);
         const bool in_seg = seg + lane < b1;
         const int tbl = in_seg ? table[seg + lane] : 0;
         const int s_tb = max(tb, seg * a.block_size);
@@ -407,7 +409,7 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
           issue(p0, p1, kr, vr, std::true_type{});
         };
         raw_t kr[U], vr[U];
-        int lim = WAVES == 1 ? min(s_te, pe) : s_te;  // chunks end at the part's end
+        int lim = WAVES == 1 ? min(s_te, pe * a.block_size) : s_te;  // chunks end at the part's end
         int p1 = min(s_tb + CH, lim);
         load_chunk(s_tb, p1, kr, vr);
         for (int p0 = s_tb; p0 < s_te;) {
@@ -463,9 +465,9 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
           p0 = p1;
           bool part_end = false;
           if (WAVES == 1 && p0 == lim) {
-            part_end = p0 == pe && p0 < te;
-            if (part_end) pe += P.pps * a.block_size;
-            lim = min(s_te, pe);
+            part_end = p0 == pe * a.block_size && p0 < te;
+            if (part_end) pe = min(pe + P.pps, b1);
+            lim = min(s_te, pe * a.block_size);
           }
           // Parts are folded in order: by the one wave through its LDS slot, or,
           // in a workgroup of several waves, by wave 0 below.
@@ -795,7 +797,7 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
     const int state_step = 4 * a.group;
     const int state_size = (2 + 4 * DT) * state_step;
     float* state = lds + grp * a.group + col;
-    int pe_page = b0 + P.pps;  // end of the current part
+    int pe_page = min(b0 + P.pps, b1);  // end of the current part
     int folded = 0;
     float m = -1e30f;  // reference max (log2 domain) of this lane's head column
     float lsum = 0.f;  // partial sum over this lane's token slots
@@ -879,7 +881,7 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
           acc[t] = Mfma16<T>::run(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pop, acc[t]);
         }
         if (WAVES == 1 && p1 == pe_page * a.block_size && p1 < te) {
-          pe_page += P.pps;
+          pe_page = min(pe_page + P.pps, b1);
           if (hcol) {
             if (folded > 0) fold_state<DT>(state, state_step, m, lsum, acc, true);
             store_state<DT>(state, state_step, m, lsum, acc);
