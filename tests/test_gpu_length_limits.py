@@ -6,7 +6,7 @@ result is that of the distinct tokens alone.
 import pytest
 import torch
 
-from test_gpu_attention import assert_close, oracle_decode
+from test_gpu_attention import assert_close, oracle_decode, oracle_prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +33,37 @@ def test_last_part_ends_with_the_row(gpu, dtype, heads, kv_heads):
     # Each of the two pages' tokens is seen 313 times.
     expected = oracle_decode(q, k, v, tables[:, :2], torch.tensor([2 * block]))
     assert_close(out, expected, dtype)
+
+
+def test_unsplit_prefill_reads_every_key_of_a_very_long_context(gpu):
+    """A tile that is not split along its keys covers the whole context: here 16
+    queries over 2^29 keys and more, of which all but the last two pages weigh
+    nothing (scores 85 lower), so the result is attention over those pages. One
+    workgroup takes 2^24 steps: several seconds."""
+    from vllm_rlt.kernels.hip_attention import dtype_code
+    from vllm_rlt.kernels._hip import library
+
+    lib = library()
+    block, heads, dim, queries, far = 128, 1, 32, 16, 2**22
+    gen = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(*shape, generator=gen) for shape in
+               [(queries, heads, dim)] + 2 * [(3, block, heads, dim)])
+    q[..., 0] = 8
+    k[0, ..., 0], k[1:, ..., 0] = -60, 0
+    q, k, v = (t.to(torch.bfloat16).to(gpu) for t in (q, k, v))
+    tables = torch.zeros(1, far + 2, dtype=torch.int32, device=gpu)
+    tables[0, far:] = torch.tensor([1, 2], dtype=torch.int32)
+    lengths = torch.tensor([(far + 2) * block], dtype=torch.int32, device=gpu)
+    cu = torch.tensor([0, queries], dtype=torch.int32, device=gpu)
+    # The workspace without room for key splits.
+    nbytes = lib.vrh_paged_prefill_workspace_bytes(1, queries, heads, dim)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+    out = torch.empty_like(q)
+    lib.check(lib.vrh_paged_prefill(
+        dtype_code(q.dtype), out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+        tables.data_ptr(), lengths.data_ptr(), cu.data_ptr(), 1, queries, queries, heads, heads,
+        dim, block, tables.shape[1], tables.stride(0), q.stride(0), q.stride(1), out.stride(0),
+        out.stride(1), *k.stride()[:3], *v.stride()[:3], workspace.data_ptr(), nbytes,
+        torch.cuda.current_stream().cuda_stream), "vrh_paged_prefill")
+    expected = oracle_prefill(q, k, v, tables[:, far:], torch.tensor([2 * block]), cu)
+    assert_close(out, expected, q.dtype)

@@ -244,7 +244,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
   int64_t seq;
   int q_begin, q_len, n, kvh, qb, split = 0;
   int tile = 0;       // tile number of the partials
-  int run = 1 << 24;  // sub-blocks of one key split
+  int run = 1 << 30;  // sub-blocks of one key split (unsplit: more than any context has)
   if (a.rank_in_kernel) {
     const Batch b = rank_batch(a);
     uint64_t hit;
