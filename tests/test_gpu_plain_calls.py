@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 def plain_call(op, gpu):
-    """A call of the module itself that allocates anew, or launches, each time."""
+    """A call of the module itself."""
     from vllm_rlt.kernels._extension import plain_calls
 
     plain = plain_calls()
@@ -29,8 +29,7 @@ def plain_call(op, gpu):
         rows = torch.randn(1024, 16, 128, device=gpu).to(torch.bfloat16)
         at = torch.arange(1024, device=gpu)
         args = (pool, pool.clone(), rows, rows, at // 16, at % 16)
-        # A queue of work, so that a launch has to wait for space in it.
-        return lambda: [plain.append(*args) for _ in range(2000)][0]
+        return lambda: plain.append(*args)
     gate = torch.randn(4096, 4096, device=gpu)
     return lambda: plain.silu(gate, gate)
 
@@ -39,8 +38,9 @@ def plain_call(op, gpu):
 def test_other_threads_run_during_a_call(gpu, op):
     """The interpreter lock is free while a call allocates and launches. The
     switch interval is far above the test's length, so that another thread gets
-    the lock only where this one gives it up; the calls allocate device memory
-    anew (milliseconds), or fill the launch queue."""
+    the lock only where this one gives it up. One call gives it up for a few
+    microseconds, in which the waiting thread may or may not wake: 50000 calls at
+    most are tried, until it has run."""
     call = plain_call(op, gpu)
     assert call() is not None
     count, stop = [0], []
@@ -53,18 +53,20 @@ def test_other_threads_run_during_a_call(gpu, op):
     thread = threading.Thread(target=other, daemon=True)
     interval = sys.getswitchinterval()
     sys.setswitchinterval(1000)
+    ran = False
     try:
         thread.start()
-        ran = 0
-        for _ in range(20):
+        for _ in range(50):
             torch.cuda.synchronize()
-            torch.cuda.empty_cache()
             before = count[0]
-            out = call()
-            ran += count[0] - before
-            del out
+            for _ in range(1000):
+                call()
+            # Nothing between these two lines but the calls lets go of the lock.
+            ran = count[0] != before
+            if ran:
+                break
     finally:
         stop.append(True)
         sys.setswitchinterval(interval)
         thread.join(5)
-    assert ran > 0
+    assert ran
