@@ -10,11 +10,12 @@
 //  * One 64-lane wavefront per (split, group of HPW q heads, row): HPW = 8, 4
 //    or 2 grouped-query heads when they divide the group (each loaded K/V
 //    vector serves all of them), else 1. Groups of 8-16 heads, and of 3, 5, 6
-//    or 7, run on the MFMA kernel below instead (one wave per kv head). A split is a run of whole
-//    pages: bps = max(min_bps, ceil(pages / kMaxSplits)) pages (at least 64
-//    tokens of a 16-bit type, 32 of fp32, at most 16 splits per row), so the partition depends only on
-//    the row's own length -> batch invariance. The split index is rotated
-//    per (row, head) so that every XCD receives the same share of splits.
+//    or 7, run on the MFMA kernel below instead (one wave per kv head). A split is
+//    a run of whole pages: at least long_bps (128 tokens of a 16-bit type, 64 of
+//    fp32), half of that in short rows (kShortSplits), at most 16 splits per row.
+//    The partition depends only on the row's own length -> batch invariance. The
+//    split index is rotated per (row, head) so that every XCD receives the same
+//    share of splits.
 //  * A longer split is a chain of up to 8 parts (4 in the MFMA kernel), folded in
 //    order. One wave runs them one after another where the launch has waves
 //    enough; launches of few splits give each split a workgroup with one wave
@@ -48,13 +49,19 @@ namespace {
 // Wave loads per chunk (in flight per lane for each of K and V), minimum and
 // maximum split length, grouped-query heads one wave may serve.
 constexpr int kMaxSplits = 16;
-// Minimum K bytes of a split (64 tokens of a 16-bit type at head_dim 128, 32 of
+// K bytes of the shortest splits (64 tokens of a 16-bit type at head_dim 128, 32 of
 // fp32), at most kSplitTokens tokens (shorter ones of head_dim 64: 18 rows of up
-// to 1757 tokens over 8 kv heads 32 against 24 us). Against 128 tokens of any type: 8 fp32 rows of
-// 64-512 tokens 14.9 against 19.4 us, 64 bf16 rows 36.6 against 39.1, 37 f16
-// rows of up to 6000 over 8 kv heads 103 against 108, 64 rows of 512-4096 the
-// same; 32 tokens of a 16-bit type were slower again (100 rows of up to 300
-// tokens 32.9 against 28.2).
+// to 1757 tokens over 8 kv heads 32 against 24 us). Rows of two to kShortSplits of
+// them are cut that finely; shorter rows are one split (64 bf16 rows of 65-128
+// tokens 11.6 us, 16.0 in two splits and a merge), longer ones have splits twice as
+// long (up to kSplitTokens). Against 128 tokens in every row: 8 fp32 rows of 64-512
+// tokens 13.8 against 19.1 us, 64 bf16 rows of 64-512 33.5 against 36.8, 8 of
+// 512-1000 15.2 against 15.5. With up to 16 short splits: 128 rows sharing 512
+// tokens 141 us, 135 with 6; 37 rows of 64-1500, 64 over 8 heads, 32.5 and 28.1;
+// with 8: 8 bf16 rows of 512-1000 15.8; with 4: 100 rows of 16-300 39.3 and 31.5.
+// What the fine splits cost: 64 fp32 rows of 65-128 tokens 23.7 us, 20.1 as one
+// split (in which the 8 fp32 rows above would take 21).
+constexpr int kShortSplits = 6;
 constexpr int kSplitBytes = 16384;
 constexpr int kSplitTokens = 128;
 constexpr int kParts = 8;           // most parts of a split (VALU kernel, MFMA kernel)
@@ -106,7 +113,8 @@ struct DecodeArgs {
   int32_t num_seqs;
   int32_t expand_e;
   int32_t q_heads, group, head_dim, block_size, bs_shift, window, min_bps, table_width;
-  int32_t long_bps;   // pages of the shortest split of rows past kMaxSplits shortest splits
+  int32_t long_bps;   // pages of the shortest split of other rows
+  int32_t short_pages;  // longest row (pages) cut into splits of min_bps
   int32_t min_part;   // pages of the shortest part of a split
   int32_t max_parts;  // most parts of a split
   float scale_log2;
@@ -131,8 +139,8 @@ __device__ __forceinline__ Partition partition(int n, const DecodeArgs& a) {
     p.first = p.start / a.block_size;
     p.pages = (n + a.block_size - 1) / a.block_size - p.first;
   }
-  p.bps = max(p.pages <= kMaxSplits * a.min_bps ? a.min_bps : a.long_bps,
-              ceil_div(p.pages, kMaxSplits));
+  const int least = p.pages > a.long_bps && p.pages <= a.short_pages ? a.min_bps : a.long_bps;
+  p.bps = max(least, ceil_div(p.pages, kMaxSplits));
   p.nsplit = ceil_div(p.pages, p.bps);
   p.pps = min(p.bps, max(a.min_part, ceil_div(p.bps, a.max_parts)));
   return p;
@@ -561,7 +569,7 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
     // Rank only when the group's split lengths differ by 2x or more: only then
     // does the order shorten the drain (and rows of equal split length, such
     // as rows sharing a prefix, keep their dispatch neighbourhood). The short
-    // splits of rows up to kMaxSplits of them count as long as long_bps pages:
+    // splits of short rows count as long as long_bps pages:
     // ranking them behind splits of twice their length took 149 us instead of
     // 142 for 128 rows in groups of 8 that share 512 tokens and have 64-1024 of
     // their own, 15.5 instead of 14.2 for 4 rows of 300-2000 (64 such rows, nothing
@@ -1196,15 +1204,12 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   a.table_width = table_width;
   a.line_shared = ((int64_t)head_dim * es) % 128 != 0;
   a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)head_dim));
-  // Pages per split: at least kSplitTokens tokens; without a workspace every
-  // row is a single split (pages can never exceed the table width).
+  // Pages per split; without a workspace every row is a single split (pages can
+  // never exceed the table width).
   const int split_tokens = std::min(kSplitTokens, kSplitBytes / (head_dim * es));
   a.min_bps = workspace != nullptr ? std::max(1, split_tokens / block_size)
                                    : std::max(1, table_width);
-
-  // Rows too long for the shortest splits: at least twice as many tokens (up to
-  // kSplitTokens), so that rows of like length, which share prefix pages, keep
-  // splits that start at the same tokens.
+  a.short_pages = workspace != nullptr ? kShortSplits * a.min_bps : 0;
   a.long_bps = std::max(a.min_bps, std::min(kSplitTokens, 2 * split_tokens) / block_size);
 
   // Grouped-query heads per wave: the largest of 8, 4, 2 dividing the group
@@ -1231,7 +1236,12 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   // Largest split count any row of this table width can need: the grid is a
   // function of shapes only (graph capture), never of device lengths.
   const int max_pages = std::max(1, table_width);
-  const int gx = std::max(1, std::min(kMaxSplits, ceil_div(max_pages, a.min_bps)));
+  // No more columns than that: 37 rows of 64-900 tokens over 8 kv heads, splits of
+  // 128 tokens, 35 us with 16 columns and 28 with 8.
+  const int gx = std::min(
+      kMaxSplits,
+      std::max(max_pages > a.long_bps ? ceil_div(std::min(max_pages, a.short_pages), a.min_bps) : 1,
+               ceil_div(max_pages, a.long_bps)));
   // Rows per launch: the grid's z limit rounded down to whole 64-row groups
   // (the longest-first ranking works on aligned groups of 64 rows).
   constexpr int64_t kRowsPerLaunch = 65535 / 64 * 64;
