@@ -16,12 +16,13 @@
 //    The partition depends only on the row's own length -> batch invariance. The
 //    split index is rotated per (row, head) so that every XCD receives the same
 //    share of splits.
-//  * A longer split is a chain of up to 8 parts (4 in the MFMA kernel), folded in
-//    order. One wave runs them one after another where the launch has waves
-//    enough; launches of few splits give each split a workgroup with one wave
-//    per part, folded through LDS in the same order: the same bits, many times
-//    the loads in flight. One row of 24001 tokens (16 x 128 heads, bf16) takes
-//    41 us instead of 78, two rows of 32 over 8 heads at 30000 42 instead of 119.
+//  * A longer split (from four shortest splits) is a chain of up to 8 parts (4 for
+//    grouped heads), folded in order. One wave runs them one after another where
+//    the launch has waves enough; launches of few splits give each split a
+//    workgroup with one wave per part, folded through LDS in the same order: the
+//    same bits, many times the loads in flight. One row of 24001 tokens (16 x 128
+//    heads, bf16) takes 40 us instead of 78, three rows of 24000 over 8 kv heads
+//    (32 heads) 54 instead of 110.
 //  * Lane layout: LPT lanes cover one token's head_dim with VEC elements each
 //    (16-byte global loads for bf16 D=128: LPT=16), so one wave-wide load
 //    instruction fetches TPL = 64 / LPT tokens; U loads of K and U of V are
@@ -64,8 +65,12 @@ constexpr int kMaxSplits = 16;
 constexpr int kShortSplits = 6;
 constexpr int kSplitBytes = 16384;
 constexpr int kSplitTokens = 128;
-constexpr int kParts = 8;           // most parts of a split (VALU kernel, MFMA kernel)
-constexpr int kMfmaParts = 4;
+// Most parts of a split for one head and for several (VALU or MFMA). Four waves of
+// several heads' state take what a CU has (two workgroups of 170-189 VGPRs); with
+// eight, 4 rows of 24000 tokens, 32 over 8 heads, took 72 us instead of 61, and
+// launches that run parts in turn fold twice as often.
+constexpr int kParts = 8;
+constexpr int kGroupParts = 4;
 constexpr int kMaxHpw = 8;
 constexpr int kU = 8;                // wave loads per chunk (K and V each)
 
@@ -117,6 +122,7 @@ struct DecodeArgs {
   int32_t short_pages;  // longest row (pages) cut into splits of min_bps
   int32_t min_part;   // pages of the shortest part of a split
   int32_t max_parts;  // most parts of a split
+  int32_t part_unit;  // pages of a chunk: parts are whole multiples
   float scale_log2;
 };
 
@@ -126,7 +132,6 @@ struct Partition {
   int pages;    // pages touched
   int bps;      // pages per split
   int nsplit;
-  int pps;      // pages per part of a split
 };
 
 __device__ __forceinline__ Partition partition(int n, const DecodeArgs& a) {
@@ -142,8 +147,19 @@ __device__ __forceinline__ Partition partition(int n, const DecodeArgs& a) {
   const int least = p.pages > a.long_bps && p.pages <= a.short_pages ? a.min_bps : a.long_bps;
   p.bps = max(least, ceil_div(p.pages, kMaxSplits));
   p.nsplit = ceil_div(p.pages, p.bps);
-  p.pps = min(p.bps, max(a.min_part, ceil_div(p.bps, a.max_parts)));
   return p;
+}
+
+// Pages per part of a split (the whole split: one part). A split shorter than two
+// shortest parts is not cut: folding costs launches that run parts in turn 4-8 % at
+// two parts (6 rows of 2300-3000 tokens, 32 over 8 heads, 27.2 against 25.6 us) and
+// gains lone rows little (19.8 against 21.5). Parts are whole chunks, so that only a
+// split's last one has a chunk that is not full (3 rows of 18000-22500 tokens 97.9
+// us without, 94.2 with).
+__device__ __forceinline__ int part_pages(const Partition& p, const DecodeArgs& a) {
+  if (p.bps < 2 * a.min_part) return p.bps;
+  const int even = ceil_div(p.bps, a.max_parts);
+  return max(a.min_part, ceil_div(even, a.part_unit) * a.part_unit);
 }
 
 __device__ __forceinline__ int clamp_length(int n, const DecodeArgs& a) {
@@ -325,7 +341,7 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
     for (int split = split0; split < P.nsplit; split += step) {
       const int s0 = P.first + split * P.bps;
       const int s1 = min(s0 + P.bps, P.first + P.pages);
-      const int parts = ceil_div(s1 - s0, P.pps);
+      const int pps = WAVES > 0 ? part_pages(P, a) : 64;
       float m[HPW], l[HPW];
       float acc[HPW][VEC];
       auto reset = [&]() {
@@ -341,19 +357,19 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
       // This wave's pages: all parts of the split, or its own one. The table is
       // read 64 pages at a time at most, whole parts where they fit, so chunks
       // start at the same tokens either way.
-      const int b0 = WAVES > 1 ? min(s0 + wave * P.pps, s1) : s0;
-      const int b1 = WAVES > 1 ? min(b0 + P.pps, s1) : s1;
+      const int b0 = WAVES > 1 ? min(s0 + wave * pps, s1) : s0;
+      const int b1 = WAVES > 1 ? min(b0 + pps, s1) : s1;
       const int tb = max(P.start, b0 * a.block_size);
       const int te = min(n, b1 * a.block_size);
-      const int seg_pages = P.pps <= 64 ? 64 / P.pps * P.pps : 64;
+      const int seg_pages = WAVES > 0 && pps <= 64 ? 64 / pps * pps : 64;
       // End of the current part (page). Never past the wave's own pages: times
       // block_size it has to stay in 32 bits for contexts close to 2^31 tokens.
-      int pe = min(b0 + P.pps, b1);
+      int pe = min(b0 + pps, b1);
       int folded = 0;
 
       for (int seg = b0, seg1; seg < b1; seg = seg1) {
         seg1 = min(b1, seg + seg_pages);
-        if (P.pps > 64) seg1 = min(seg1, pe);
+        if (WAVES > 0 && pps > 64) seg1 = min(seg1, pe);
         const bool in_seg = seg + lane < b1;
         const int tbl = in_seg ? table[seg + lane] : 0;
         const int s_tb = max(tb, seg * a.block_size);
@@ -417,10 +433,7 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
           issue(p0, p1, kr, vr, std::true_type{});
         };
         raw_t kr[U], vr[U];
-        int lim = WAVES == 1 ? min(s_te, pe * a.block_size) : s_te;  // chunks end at the part's end
-        int p1 = min(s_tb + CH, lim);
-        load_chunk(s_tb, p1, kr, vr);
-        for (int p0 = s_tb; p0 < s_te;) {
+        auto attend = [&](int p0, int p1) {
           float sc[HPW][U];
           float mx[HPW];
 #pragma unroll
@@ -470,34 +483,59 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
           }
 #pragma unroll
           for (int h = 0; h < HPW; ++h) m[h] = mx[h];
-          p0 = p1;
-          bool part_end = false;
-          if (WAVES == 1 && p0 == lim) {
-            part_end = p0 == pe * a.block_size && p0 < te;
-            if (part_end) pe = min(pe + P.pps, b1);
+        };
+        auto end_part = [&]() {
+          if (folded > 0) fold_state<HPW, VEC>(lds, lane, m, l, acc, true);
+          store_state<HPW, VEC>(lds, lane, m, l, acc);
+          reset();
+          ++folded;
+        };
+        // Chunks end at lim: the end of the part (WAVES 1) or of the table segment.
+        // Parts are folded in order: by the one wave through its LDS slot, or, in a
+        // workgroup of several waves, by wave 0 below.
+        int p0 = s_tb;
+        int lim = WAVES == 1 ? min(s_te, pe * a.block_size) : s_te;
+        load_chunk(p0, min(p0 + CH, lim), kr, vr);
+        if constexpr (WAVES == 1 && HPW == 1) {
+          // One head: the next chunk's loads go out before the fold.
+          while (p0 < s_te) {
+            const int p1 = min(p0 + CH, lim);
+            attend(p0, p1);
+            p0 = p1;
+            bool part_end = false;
+            if (p0 == lim) {
+              part_end = p0 == pe * a.block_size && p0 < te;
+              if (part_end) pe = min(pe + pps, b1);
+              lim = min(s_te, pe * a.block_size);
+            }
+            if (p0 < s_te) load_chunk(p0, min(p0 + CH, lim), kr, vr);
+            if (part_end) end_part();
+          }
+        } else {
+          // Several heads: their state leaves no registers for loads in flight across
+          // the fold, and the chunk loop must not pay for it.
+          while (true) {
+            for (; p0 < lim; p0 += CH) {
+              const int p1 = min(p0 + CH, lim);
+              attend(p0, p1);
+              if (p1 < lim) load_chunk(p1, min(p1 + CH, lim), kr, vr);
+            }
+            if constexpr (WAVES != 1) break;
+            p0 = lim;
+            if (p0 == pe * a.block_size && p0 < te) {
+              end_part();
+              pe = min(pe + pps, b1);
+            }
             lim = min(s_te, pe * a.block_size);
+            if (p0 >= lim) break;
+            load_chunk(p0, min(p0 + CH, lim), kr, vr);
           }
-          // Parts are folded in order: by the one wave through its LDS slot, or,
-          // in a workgroup of several waves, by wave 0 below.
-          auto end_part = [&]() {
-            if (folded > 0) fold_state<HPW, VEC>(lds, lane, m, l, acc, true);
-            store_state<HPW, VEC>(lds, lane, m, l, acc);
-            reset();
-            ++folded;
-          };
-          // One head: the next chunk's loads go out before the fold. Several:
-          // their registers are not free until after it.
-          if (WAVES == 1 && HPW > 1 && part_end) end_part();
-          if (p0 < s_te) {
-            p1 = min(p0 + CH, lim);
-            load_chunk(p0, p1, kr, vr);
-          }
-          if (WAVES == 1 && HPW == 1 && part_end) end_part();
         }
       }
       if (WAVES == 1 && folded > 0) fold_state<HPW, VEC>(lds, lane, m, l, acc, true);
       if constexpr (WAVES > 1) {
         constexpr int kSlot = HPW * (VEC + 2) * 64;
+        const int parts = ceil_div(s1 - s0, pps);
         if (wave > 0 && wave < parts) store_state<HPW, VEC>(lds + (wave - 1) * kSlot, lane, m, l, acc);
         __syncthreads();
         if (wave > 0) return;
@@ -600,16 +638,23 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
 }
 
 // Splits of a launch up to which each split gets a workgroup, one wave a part:
-// with more, single waves fill the chip by themselves. VALU kernel: 2 rows of
-// 24000 tokens (512 splits) 74 against 95 us, 4 rows of 4000 (1024) 34 against
-// 30. MFMA kernel (8 kv heads): 6 rows of 24000 (768) 128 against 140, 8 rows of
-// 4000-8000 (1024) 55 against 58.
-constexpr int kWideSplits = 512;
-constexpr int kWideMfmaSplits = 1024;
+// with more, single waves fill the chip by themselves. One head per wave, bf16 /
+// fp32, at 768 (3 rows of 24000 tokens) 79.4 / 147 us against 82.8 / 158 in turn, at
+// 1024 (4 rows of 3000) 25.4 / 33.7 against 21.0 / 32.5. Several heads: four parts
+// at 1536 (12 rows of 24000, 32 over 8 heads) 171 against 197, at 2048 (16 rows of
+// 18000-24000) 274 against 248; with two parts two of the four waves idle (6 rows of
+// 3000, 768 splits, 36 against 27). Eight heads per wave, 16 over 2 of dim 32: 6
+// rows of 24000 (768) 85 against 76. MFMA kernel (8 kv heads): 6 rows of 24000
+// (768) 108 against 124, 8 rows of 8000 (1024) 49 against 46.
+constexpr int kWideSplits = 768;
+constexpr int kWideMfmaSplits = 768;
+constexpr int kWideGroupSplits = 1536;  // two or four heads per wave, more than two parts
+constexpr int kWideFewSplits = 512;     // otherwise
 
 // Grid form: one wave per (split column, group of HPW q heads, row).
 template <typename T, int VEC, int LPT, int HPW, int WAVES>
-__global__ __launch_bounds__(WAVES > 1 ? 64 * WAVES : 64) void paged_decode_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(WAVES > 1 ? 64 * WAVES : 64)
+void paged_decode_kernel(DecodeArgs a) {
   constexpr int kSlots = WAVES > 1 ? WAVES - 1 : WAVES;
   __shared__ float state[kSlots > 0 ? kSlots * HPW * (VEC + 2) * 64 : 1];
   int64_t row;
@@ -797,15 +842,16 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
     // Parts of the split as in decode_work: all of them, or this wave's one.
     const int s0 = P.first + split * P.bps;
     const int s1 = min(s0 + P.bps, P.first + P.pages);
-    const int b0 = WAVES > 1 ? min(s0 + wave * P.pps, s1) : s0;
-    const int b1 = WAVES > 1 ? min(b0 + P.pps, s1) : s1;
+    const int pps = WAVES > 0 ? part_pages(P, a) : 64;
+    const int b0 = WAVES > 1 ? min(s0 + wave * pps, s1) : s0;
+    const int b1 = WAVES > 1 ? min(b0 + pps, s1) : s1;
     const int tb = max(P.start, b0 * a.block_size);
     const int te = min(n, b1 * a.block_size);
-    const int seg_pages = P.pps <= 64 ? 64 / P.pps * P.pps : 64;
+    const int seg_pages = WAVES > 0 && pps <= 64 ? 64 / pps * pps : 64;
     const int state_step = 4 * a.group;
     const int state_size = (2 + 4 * DT) * state_step;
     float* state = lds + grp * a.group + col;
-    int pe_page = min(b0 + P.pps, b1);  // end of the current part
+    int pe = min(b0 + pps, b1);  // end of the current part (page)
     int folded = 0;
     float m = -1e30f;  // reference max (log2 domain) of this lane's head column
     float lsum = 0.f;  // partial sum over this lane's token slots
@@ -815,81 +861,85 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
 
     for (int seg = b0, seg1; seg < b1; seg = seg1) {
       seg1 = min(b1, seg + seg_pages);
-      if (P.pps > 64) seg1 = min(seg1, pe_page);
+      if (WAVES > 0 && pps > 64) seg1 = min(seg1, pe);
       const int tbl = (seg + lane < b1) ? table[seg + lane] : 0;
       const int s_tb = max(tb, seg * a.block_size);
       const int s_te = min(te, seg1 * a.block_size);
-      for (int p0 = s_tb, p1; p0 < s_te; p0 = p1) {
-        // Chunks end at the part's end.
-        p1 = min(min(p0 + kMfmaChunk, s_te), pe_page * a.block_size);
-        // Loads (branch-free: positions past the end re-read the last token).
-        // The A-operand layout gives each token 4 lanes (64 bytes) per
-        // instruction, so instructions c and c + 1 read the two halves of one
-        // 128-byte line: ordinary (L1-allocating) loads let the second half
-        // hit the line the first brought in.
-        u32x4_t kop[2][DC];
+      // Chunks end at lim: the end of the part (WAVES 1) or of the table segment.
+      int p0 = s_tb;
+      do {
+        const int lim = WAVES == 1 ? min(s_te, pe * a.block_size) : s_te;
+        for (; p0 < lim; p0 += kMfmaChunk) {
+          // Loads (branch-free: positions past the end re-read the last token).
+          // The A-operand layout gives each token 4 lanes (64 bytes) per
+          // instruction, so instructions c and c + 1 read the two halves of one
+          // 128-byte line: ordinary (L1-allocating) loads let the second half
+          // hit the line the first brought in.
+          u32x4_t kop[2][DC];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int pos = min(p0 + 16 * t + col, p1 - 1);
-          const T* kp = kbase + page_addr(pos, tbl, seg, a.k_block, a.k_token);
+          for (int t = 0; t < 2; ++t) {
+            const int pos = min(p0 + 16 * t + col, lim - 1);
+            const T* kp = kbase + page_addr(pos, tbl, seg, a.k_block, a.k_token);
 #pragma unroll
-          for (int c = 0; c < DC; ++c) kop[t][c] = *reinterpret_cast<const u32x4_t*>(kp + 32 * c);
-        }
-        // V straight into the LDS tile. The previous chunk's transposed reads
-        // have returned (its PV MFMAs consumed them), so the tile is free.
-#pragma unroll
-        for (int r = 0; r < NV; ++r) {
-          const int pos = min(p0 + v_row + RPI * r, p1 - 1);
-          const T* vp = vbase[r % SWP] + page_addr(pos, tbl, seg, a.v_block, a.v_token);
-          lds_dma16(vp, __builtin_amdgcn_readfirstlane(vt_lds + 1024 * r));
-        }
-        // S tiles and their masked max (tokens p0 + 16t + 4grp + i).
-        f32x4_t sc[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          sc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int c = 0; c < DC; ++c) sc[t] = Mfma16<T>::run(kop[t][c], qop[c], sc[t]);
-        }
-        const int lim = p1 - p0 - 4 * grp;  // token slot t*16 + i visible when < lim
-        float mx = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float x = 16 * t + i < lim ? sc[t][i] * a.scale_log2 : -INFINITY;
-            sc[t][i] = x;
-            mx = fmaxf(mx, x);
+            for (int c = 0; c < DC; ++c) kop[t][c] = *reinterpret_cast<const u32x4_t*>(kp + 32 * c);
           }
-        mx = fmaxf(mx, shfl_xor_f32(mx, 16));
-        mx = fmaxf(mx, shfl_xor_f32(mx, 32));
-        if (__any(mx > m + 8.f)) {
-          const float mnew = fmaxf(m, mx);
-          const float corr = fast_exp2(m - mnew);
-          lsum *= corr;
+          // V straight into the LDS tile. The previous chunk's transposed reads
+          // have returned (its PV MFMAs consumed them), so the tile is free.
 #pragma unroll
-          for (int t = 0; t < DT; ++t) acc[t] *= corr;
-          m = mnew;
-        }
-        float p[2][4];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            p[t][i] = fast_exp2(sc[t][i] - m);
-            lsum += p[t][i];
+          for (int r = 0; r < NV; ++r) {
+            const int pos = min(p0 + v_row + RPI * r, lim - 1);
+            const T* vp = vbase[r % SWP] + page_addr(pos, tbl, seg, a.v_block, a.v_token);
+            lds_dma16(vp, __builtin_amdgcn_readfirstlane(vt_lds + 1024 * r));
           }
-        const u32x4_t pop = u32x4_t{pack2<T>(p[0][0], p[0][1]), pack2<T>(p[0][2], p[0][3]),
-                                    pack2<T>(p[1][0], p[1][1]), pack2<T>(p[1][2], p[1][3])};
-        vm_wait<0>();  // the V tile has landed
+          // S tiles and their masked max (tokens p0 + 16t + 4grp + i).
+          f32x4_t sc[2];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) {
-          const u32x2_t lo = lds_tr16(vt + tr_off[t]);
-          const u32x2_t hi = lds_tr16(vt + tr_off[t] + 16 * D);
-          acc[t] = Mfma16<T>::run(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pop, acc[t]);
+          for (int t = 0; t < 2; ++t) {
+            sc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < DC; ++c) sc[t] = Mfma16<T>::run(kop[t][c], qop[c], sc[t]);
+          }
+          const int left = lim - p0 - 4 * grp;  // token slot t*16 + i visible when < left
+          float mx = -INFINITY;
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float x = 16 * t + i < left ? sc[t][i] * a.scale_log2 : -INFINITY;
+              sc[t][i] = x;
+              mx = fmaxf(mx, x);
+            }
+          mx = fmaxf(mx, shfl_xor_f32(mx, 16));
+          mx = fmaxf(mx, shfl_xor_f32(mx, 32));
+          if (__any(mx > m + 8.f)) {
+            const float mnew = fmaxf(m, mx);
+            const float corr = fast_exp2(m - mnew);
+            lsum *= corr;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) acc[t] *= corr;
+            m = mnew;
+          }
+          float p[2][4];
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              p[t][i] = fast_exp2(sc[t][i] - m);
+              lsum += p[t][i];
+            }
+          const u32x4_t pop = u32x4_t{pack2<T>(p[0][0], p[0][1]), pack2<T>(p[0][2], p[0][3]),
+                                      pack2<T>(p[1][0], p[1][1]), pack2<T>(p[1][2], p[1][3])};
+          vm_wait<0>();  // the V tile has landed
+#pragma unroll
+          for (int t = 0; t < DT; ++t) {
+            const u32x2_t lo = lds_tr16(vt + tr_off[t]);
+            const u32x2_t hi = lds_tr16(vt + tr_off[t] + 16 * D);
+            acc[t] = Mfma16<T>::run(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pop, acc[t]);
+          }
         }
-        if (WAVES == 1 && p1 == pe_page * a.block_size && p1 < te) {
-          pe_page = min(pe_page + P.pps, b1);
+        p0 = lim;
+        if (WAVES == 1 && lim == pe * a.block_size && lim < te) {
+          pe = min(pe + pps, b1);
           if (hcol) {
             if (folded > 0) fold_state<DT>(state, state_step, m, lsum, acc, true);
             store_state<DT>(state, state_step, m, lsum, acc);
@@ -900,11 +950,11 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
           for (int t = 0; t < DT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
           ++folded;
         }
-      }
+      } while (p0 < s_te);
     }
     if (folded > 0 && hcol) fold_state<DT>(state, state_step, m, lsum, acc, true);
     if constexpr (WAVES > 1) {
-      const int parts = ceil_div(s1 - s0, P.pps);
+      const int parts = ceil_div(s1 - s0, pps);
       if (wave > 0 && wave < parts && hcol)
         store_state<DT>(state + (wave - 1) * state_size, state_step, m, lsum, acc);
       __syncthreads();
@@ -936,11 +986,15 @@ __device__ __forceinline__ void decode_work_mfma(const DecodeArgs& a, int64_t ro
   }
 }
 
-// Dynamic LDS: mfma_state_bytes per state (one, or WAVES - 1).
+// Dynamic LDS: mfma_state_bytes per state (one, or WAVES - 1). Single waves: three
+// per SIMD at head_dim 128 and four at 64, also where registers would allow more
+// (40 rows of 6000-8000 tokens, 64 over 8 heads of dim 64: 146 us with six, 134
+// with four).
 template <typename T, int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 ? 3 : 2)))
+__global__ __launch_bounds__(WAVES > 1 ? 64 * WAVES : 64)
+__attribute__((amdgpu_waves_per_eu(WAVES > 1 ? 2 : D == 128 ? 3 : 4, WAVES > 1 ? 8 : D == 128 ? 3 : 4)))
 void paged_decode_mfma_kernel(DecodeArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t vt[WAVES][kMfmaChunk * D];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[WAVES > 1 ? WAVES : 1][kMfmaChunk * D];
   extern __shared__ float mfma_state[];
   int64_t row;
   int split0;
@@ -959,8 +1013,10 @@ void launch_mfma(int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
   const size_t state = mfma_state_bytes(D, a.group);
   if (waves > 1)
     hipLaunchKernelGGL((paged_decode_mfma_kernel<T, D, 4>), grid, dim3(256), 3 * state, s, a);
+  else if (waves == 1)
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<T, D, 1>), grid, dim3(64), state, s, a);
   else
-    hipLaunchKernelGGL((paged_decode_mfma_kernel<T, D, 1>), grid, dim3(64), waves > 0 ? state : 0, s, a);
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<T, D, 0>), grid, dim3(64), 0, s, a);
 }
 
 // Log-sum-exp merge of one (row, q head)'s split partials by one wave, for
@@ -1035,9 +1091,13 @@ void launch_merge(int head_dim, dim3 grid, hipStream_t s, const DecodeArgs& a) {
 
 template <typename T, int VEC, int LPT, int HPW>
 void launch_waves(int waves, dim3 grid, hipStream_t s, const DecodeArgs& a) {
-  if (waves == 8)
-    hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 8>), grid, dim3(512), 0, s, a);
-  else if (waves == 4)
+  if constexpr (HPW == 1) {
+    if (waves == 8) {
+      hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 8>), grid, dim3(512), 0, s, a);
+      return;
+    }
+  }
+  if (waves == 4)
     hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 4>), grid, dim3(256), 0, s, a);
   else if (waves == 1)
     hipLaunchKernelGGL((paged_decode_kernel<T, VEC, LPT, HPW, 1>), grid, dim3(64), 0, s, a);
@@ -1231,8 +1291,10 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
                         a.group <= kMfmaHeads && (a.group >= kMfmaAllGroups || hpw < a.group);
   // Other lane layouts have no workgroups of several waves, so no parts either.
   const bool has_parts = vec * es == 16 && lpt >= 4 && lpt <= 32;
-  a.min_part = has_parts ? 2 * a.min_bps : 1 << 30;
-  a.max_parts = mfma_gqa ? kMfmaParts : kParts;
+  a.min_part = has_parts ? 2 * a.min_bps : 1 << 29;
+  a.max_parts = mfma_gqa || hpw > 1 ? kGroupParts : kParts;
+  const int chunk = mfma_gqa ? kMfmaChunk : std::min(kU, std::max(1, 2 * kU / hpw)) * (64 / lpt);
+  a.part_unit = std::max(1, chunk / block_size);
   // Largest split count any row of this table width can need: the grid is a
   // function of shapes only (graph capture), never of device lengths.
   const int max_pages = std::max(1, table_width);
@@ -1253,11 +1315,16 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
     // have, and whether each gets a workgroup (kWideSplits).
     const int seen_pages =
         window > 0 ? (int)std::min<int64_t>(max_pages, (int64_t)window / block_size + 2) : max_pages;
-    const int parts =
-        std::min(a.max_parts, ceil_div(std::max(a.long_bps, ceil_div(seen_pages, kMaxSplits)), a.min_part));
+    const int longest = std::max(a.long_bps, ceil_div(seen_pages, kMaxSplits));
+    const int parts = longest < 2 * a.min_part
+                          ? 1
+                          : std::min(a.max_parts, ceil_div(longest, a.min_part));
     const int units = mfma_gqa ? kv_heads : q_heads / hpw;
-    const bool wide =
-        parts > 1 && (int64_t)gx * units * count <= (mfma_gqa ? kWideMfmaSplits : kWideSplits);
+    const int widest = mfma_gqa               ? kWideMfmaSplits
+                       : hpw == 1             ? kWideSplits
+                       : hpw < 8 && parts > 2 ? kWideGroupSplits
+                                              : kWideFewSplits;
+    const bool wide = parts > 1 && (int64_t)gx * units * count <= widest;
     const int waves = parts <= 1 ? 0 : !wide ? 1 : parts > 4 ? 8 : 4;
     const dim3 grid((unsigned)gx, (unsigned)units, count);
     if (mfma_gqa) {
