@@ -68,6 +68,32 @@ def test_split_tiles_match_oracle(gpu, batch, dtype, heads, kv_heads, head_dim):
     assert_close(call(lib, inputs, full - 1), expected, dtype)
 
 
+@pytest.mark.parametrize("sequences,split", [
+    ([(40, 40), (30, 30), (1300, 1), (17, 1)], False),  # wide tables, nothing to split
+    ([(1200, 40), (30, 30), (90, 1), (17, 1)], True),
+    ([(1300, 1), (20, 1), (3, 3), (60, 20)], False)])
+@pytest.mark.parametrize("dtype,heads,kv_heads,head_dim", [
+    (torch.bfloat16, 8, 8, 128), (torch.float16, 6, 2, 64), (torch.bfloat16, 2, 1, 32)])
+def test_decode_rows_merged_beside_the_tiles(gpu, sequences, split, dtype, heads, kv_heads,
+                                             head_dim):
+    """One launch merges the split decode rows and the tiles' key splits: the rows'
+    bits are those of a call without key splits, and the tiles' too where no tile
+    turns out to be split."""
+    from vllm_rlt.kernels._hip import library
+
+    lib = library()
+    inputs = prefill_inputs(sequences, heads, kv_heads, head_dim, dtype, gpu, seed=11)
+    base, full = sizes(lib, inputs)
+    assert full > base
+    merged, unsplit = call(lib, inputs, full), call(lib, inputs, base)
+    assert_close(merged, oracle_prefill(*inputs[:6]), dtype)
+    at = 0
+    for _, queries in sequences:
+        if queries == 1 or not split:
+            assert torch.equal(merged[at : at + queries], unsplit[at : at + queries])
+        at += queries
+
+
 def test_split_prefill_in_a_graph_follows_the_device_lengths(gpu):
     """Captured once with wide tables, replayed after the lengths changed: the
     runs come from the device lengths, the grid only from the shapes."""

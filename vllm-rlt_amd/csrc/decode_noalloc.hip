@@ -17,18 +17,7 @@
 // concurrently) share the array and race.
 #include <mutex>
 
-#include "common.h"
-
-int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
-                    const void* value_cache, const int32_t* block_tables,
-                    const int32_t* context_lengths, const int32_t* cu_q, int32_t num_seqs,
-                    int32_t expand_e, int64_t rows, int32_t q_heads, int32_t kv_heads,
-                    int32_t head_dim, int32_t block_size, int32_t table_width,
-                    int64_t table_stride, int64_t q_row_stride, int64_t q_head_stride,
-                    int64_t out_row_stride, int64_t out_head_stride, int64_t k_block_stride,
-                    int64_t k_token_stride, int64_t k_head_stride, int64_t v_block_stride,
-                    int64_t v_token_stride, int64_t v_head_stride, int32_t window,
-                    void* workspace, size_t workspace_bytes, hipStream_t s, const char* who);
+#include "decode_rows.h"
 
 static __device__ __align__(256) unsigned char scratch[VRH_PAGED_DECODE_NOALLOC_MAX_BYTES];
 

@@ -35,18 +35,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.h"
-
-int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
-                    const void* value_cache, const int32_t* block_tables,
-                    const int32_t* context_lengths, const int32_t* cu_q, int32_t num_seqs,
-                    int32_t expand_e, int64_t rows, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
-                    int32_t block_size, int32_t table_width, int64_t table_stride,
-                    int64_t q_row_stride, int64_t q_head_stride, int64_t out_row_stride,
-                    int64_t out_head_stride, int64_t k_block_stride, int64_t k_token_stride,
-                    int64_t k_head_stride, int64_t v_block_stride, int64_t v_token_stride,
-                    int64_t v_head_stride, int32_t window, void* workspace,
-                    size_t workspace_bytes, hipStream_t s, const char* who);
+#include "decode_rows.h"
 
 namespace vrh {
 namespace {
@@ -106,6 +95,7 @@ struct PrefillArgs {
   int32_t target;             // workgroups the key splits aim at
   float* part_acc;            // [tile, kv head, split][wave][d block][4][64 lanes][4]
   float* part_ml;             // [tile, kv head, split][wave][32 queries][2]
+  int32_t* any_split;         // whether any tile has more than one run (set by the first workgroup)
   int32_t group, block_size, bs_shift, table_width;
   int32_t skip_q;  // sequences with q_len <= skip_q are left to the decode kernel
   int32_t uniform_pages;  // block size a power-of-two multiple of 256 / (16-byte chunks per row)
@@ -247,6 +237,10 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
   int run = 1 << 30;  // sub-blocks of one key split (unsplit: more than any context has)
   if (a.rank_in_kernel) {
     const Batch b = rank_batch(a);
+    if (a.splits > 1) {
+      run = split_run(b, a);
+      if (blockIdx.x == 0 && threadIdx.x == 0) *a.any_split = b.longest > run;
+    }
     uint64_t hit;
     if (a.compact) {
       // kv_heads a multiple of 8: kv heads fastest over the numbered tiles, so
@@ -277,7 +271,6 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
     const int before = __builtin_amdgcn_readlane(b.before, pick);
     if (!a.compact) tile += before;
     qb = __builtin_amdgcn_readlane(b.tiles, pick) - 1 - (tile - before);
-    if (a.splits > 1) run = split_run(b, a);
   } else {
     const int64_t slot = blockIdx.x / 8;
     const int64_t g = (slot / a.qblocks) * 8 + blockIdx.x % 8;
@@ -714,18 +707,30 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu))) void paged_prefil
 
 // Log-sum-exp merge of a tile's key splits, in split order. One workgroup per
 // (32 query rows, 32 dims) of a tile, one wave per 8 dims: every load is 1 KiB
-// contiguous, and kAhead splits' loads are in flight together.
+// contiguous, and kAhead splits' loads are in flight together. The first
+// decode_blocks workgroups merge the batch's decode rows instead: only the device
+// knows whether any tile was split, and a launch for that alone cost batches of
+// short prompts and long decode rows 3-10 us (8 prompts of 16-64 queries and 4 rows
+// of 3000-4000 tokens 42.9 us, 34.5 without splits and in one launch).
 template <typename T, int D>
-__global__ __launch_bounds__(256) void paged_prefill_merge_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256) void paged_prefill_merge_kernel(PrefillArgs a, DecodeArgs rows,
+                                                                  int decode_blocks) {
   constexpr int DB = D / 32;
   constexpr int kAhead = 4;
   const int lane = threadIdx.x & 63;
   const int gi = threadIdx.x >> 6;
   const int col = lane & 31, half = lane >> 5;
-  const int db = blockIdx.x % DB;
-  const int wave = blockIdx.x / DB % kWaves;  // the tile's 32-row group
-  const int tile = blockIdx.x / (DB * kWaves) / a.kv_heads;
-  const int kvh = blockIdx.x / (DB * kWaves) % a.kv_heads;
+  if ((int)blockIdx.x < decode_blocks) {
+    const int per_row = ceil_div(rows.q_heads, 4);
+    decode_merge<T, (D + 63) / 64>(rows, (int)blockIdx.x % per_row, (int)blockIdx.x / per_row);
+    return;
+  }
+  if (*a.any_split == 0) return;
+  const int item = (int)blockIdx.x - decode_blocks;
+  const int db = item % DB;
+  const int wave = item / DB % kWaves;  // the tile's 32-row group
+  const int tile = item / (DB * kWaves) / a.kv_heads;
+  const int kvh = item / (DB * kWaves) % a.kv_heads;
   const Batch b = rank_batch(a);
   const uint64_t hit = __ballot(tile >= b.before && tile < b.before + b.tiles);
   if (hit == 0) return;
@@ -783,11 +788,14 @@ __global__ __launch_bounds__(256) void paged_prefill_merge_kernel(PrefillArgs a)
 }
 
 template <typename T>
-bool launch_prefill_merge(int d, dim3 grid, hipStream_t s, const PrefillArgs& a) {
+bool launch_prefill_merge(int d, unsigned tile_blocks, hipStream_t s, const PrefillArgs& a,
+                          const DecodeArgs& rows, unsigned decode_blocks) {
+  const dim3 grid(tile_blocks + decode_blocks);
   switch (d) {
 #define VRH_D(DV)                                                                               \
   case DV:                                                                                      \
-    hipLaunchKernelGGL((paged_prefill_merge_kernel<T, DV>), grid, dim3(256), 0, s, a);          \
+    hipLaunchKernelGGL((paged_prefill_merge_kernel<T, DV>), grid, dim3(256), 0, s, a, rows,     \
+                       (int)decode_blocks);                                                     \
     return true;
     VRH_D(32)
     VRH_D(64)
@@ -1052,6 +1060,7 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
   a.cap_tiles = (int32_t)std::min<int64_t>(cap_tiles, 1 << 30);
   a.target = target_items(head_dim);
   a.part_acc = a.part_ml = nullptr;
+  a.any_split = nullptr;
   if (route_decode) {
     const size_t base =
         (vrh_paged_prefill_workspace_bytes(num_seqs, max_seqlen_q, q_heads, head_dim) + 255) / 256 * 256;
@@ -1063,6 +1072,9 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
       a.rank_in_kernel = 1;  // the runs follow from the same per-lane lengths
       a.part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + base);
       a.part_ml = a.part_acc + slots * kBM * head_dim;
+      // In the dispatch order's place, which a batch ranked in the kernel does not use.
+      a.any_split = reinterpret_cast<int32_t*>(
+          static_cast<char*>(workspace) + decode_part_bytes(num_seqs, max_seqlen_q, q_heads, head_dim));
     }
   }
   a.compact = a.rank_in_kernel && kv_heads % 8 == 0;
@@ -1086,12 +1098,9 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
                         ? launch_prefill<bf16_t>(head_dim, dim3((unsigned)launched), s, a)
                         : launch_prefill<f16_t>(head_dim, dim3((unsigned)launched), s, a);
     VRH_CHECK_ARG(ok, "vrh_paged_prefill: no kernel for head_dim %d", head_dim);
-    if (a.splits > 1) {
-      const dim3 mgrid((unsigned)(head_dim / 32 * kWaves * cap_tiles * kv_heads));
-      if (dtype == VRH_DTYPE_BF16) launch_prefill_merge<bf16_t>(head_dim, mgrid, s, a);
-      else launch_prefill_merge<f16_t>(head_dim, mgrid, s, a);
-    }
   }
+  DecodeArgs rows = {};  // merged with the tiles' runs when the call may have any
+  unsigned decode_blocks = 0;
   if (route_rows) {
     // Short sequences of the packed batch: one split-KV decode row per query
     // (row r is query r % route_q of sequence r / route_q).
@@ -1101,8 +1110,16 @@ extern "C" int vrh_paged_prefill(int dtype, void* out, const void* q, const void
         block_size, table_width, table_stride, q_token_stride, q_head_stride, out_token_stride,
         out_head_stride, k_block_stride, k_token_stride, k_head_stride, v_block_stride,
         v_token_stride, v_head_stride, 0, workspace,
-        decode_part_bytes(num_seqs, max_seqlen_q, q_heads, head_dim), s, "vrh_paged_prefill");
+        decode_part_bytes(num_seqs, max_seqlen_q, q_heads, head_dim), s, "vrh_paged_prefill",
+        a.splits > 1 ? &rows : nullptr, &decode_blocks);
     if (rc != VRH_OK) return rc;
+  }
+  if (a.splits > 1) {
+    const unsigned tile_blocks = (unsigned)(head_dim / 32 * kWaves * cap_tiles * kv_heads);
+    if (dtype == VRH_DTYPE_BF16)
+      launch_prefill_merge<bf16_t>(head_dim, tile_blocks, s, a, rows, decode_blocks);
+    else
+      launch_prefill_merge<f16_t>(head_dim, tile_blocks, s, a, rows, decode_blocks);
   }
   VRH_RETURN_LAUNCH("vrh_paged_prefill");
 }
