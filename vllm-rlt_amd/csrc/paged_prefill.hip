@@ -48,6 +48,13 @@ constexpr int kSB = 32;                    // keys per sub-block (one pipeline s
 constexpr int kStages = 3;                 // LDS stages: one sub-block each
 constexpr int kTableSeg = 512;             // page ids staged in LDS at a time
 constexpr int kMinRun = 8;                 // sub-blocks of the shortest key split
+// Sub-blocks that splitting must take off the longest tile to pay for the merge
+// launch and the partials: 4 chunks of up to 512 queries without a prefix (16
+// sub-blocks, 416 tiles) took 36 us split in two against 26 us whole, one such
+// chunk (64 tiles) 18.1 against 19.5 us. Asked of the table's width by the host and
+// of the lengths on the device: 9 prompts of 34-251 queries beside decode rows of up
+// to 4096 tokens (14 sub-blocks, head_dim 64) took 38 us split, 32 whole.
+constexpr int kMinSaved = 12;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
@@ -199,8 +206,11 @@ __device__ __forceinline__ Batch rank_batch(const PrefillArgs& a) {
 __device__ __forceinline__ int split_run(const Batch& b, const PrefillArgs& a) {
   // A tile's last run is shorter: leave room for one such run per tile.
   const int items = max(a.target - b.all_tiles * a.kv_heads, a.target / 4);
-  const int run = (int)min(((int64_t)b.work * a.kv_heads + items - 1) / items, (int64_t)1 << 24);
-  return max(max(kMinRun, run), ceil_div(b.longest, a.splits));
+  const int even = (int)min(((int64_t)b.work * a.kv_heads + items - 1) / items, (int64_t)1 << 24);
+  const int run = max(max(kMinRun, even), ceil_div(b.longest, a.splits));
+  // The host's test (kMinSaved) with the tiles and lengths that the batch has.
+  const int idle = a.target - b.all_tiles * a.kv_heads;
+  return (int64_t)b.longest * idle < (int64_t)kMinSaved * a.target ? max(run, b.longest) : run;
 }
 
 // Page addressing modes: kDiv (any block size), kShift (power of two).
@@ -902,12 +912,6 @@ constexpr int kCus = 256;
 int target_items(int32_t head_dim) { return kCus * (head_dim <= 64 ? 4 : kWgPerCu); }
 constexpr int kMaxSlots = 1536;     // partials held (68 KB each at head_dim 128)
 constexpr int kMaxKeySplits = 16;
-// Sub-blocks that splitting must take off the longest tile to pay for the merge
-// launch and the partials: 4 chunks of up to 512 queries without a prefix (16
-// sub-blocks, 416 tiles) took 36 us split in two against 26 us whole, one such
-// chunk (64 tiles) 18.1 against 19.5 us.
-constexpr int kMinSaved = 12;
-
 // Head dims of the MFMA tiles (16-bit types, 16-byte aligned rows).
 bool tile_head_dim(int32_t head_dim) { return head_dim >= 32 && head_dim <= 128 && head_dim % 32 == 0; }
 
