@@ -176,6 +176,9 @@ def test_prefill_split_workspace_follows_the_shapes():
     assert extra(4, 8, 8, 16, 16, 128, 16, 512) == 0                  # decode rows
     assert extra(65, 650, 10, 4, 4, 128, 16, 512) == 0                # not ranked in the kernel
     assert extra(1, 0, 512, 16, 16, 128, 16, 448) == 0
+    # 576 keys repay the partials of one chunk, not those of four.
+    assert extra(1, 200, 200, 16, 16, 128, 16, 36) > 0
+    assert extra(4, 800, 200, 16, 16, 128, 16, 36) == 0
     for dim in (0, 16, 80, 160, 256):  # no MFMA tiles, so no partials
         assert extra(1, 512, 512, 16, 16, dim, 16, 448) == 0
     assert extra(1, 512, 512, 4, 8, 128, 16, 448) == 0  # fewer query heads than KV heads

@@ -1,5 +1,5 @@
 // What the decode rows' kernels and the packed-prefill entry share: the arguments
-// and partition of a row, and the merge of its split partials.
+// and partition of a row, wave reductions, and the merge of its split partials.
 #pragma once
 
 #include "common.h"
@@ -117,6 +117,27 @@ __device__ __forceinline__ int row_length(int64_t row, const DecodeArgs& a, int6
   *table_row = seq;
   *query_row = a.cu_q[seq] + i;
   return clamp_length(a.lengths[seq] - q_len + i + 1, a);
+}
+
+// Maximum of an int over the wave: DPP within rows of 16 lanes, then the 4
+// row results through scalar reads (no LDS traffic).
+__device__ __forceinline__ int wave_max_i(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppQuadXor1, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppQuadXor2, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppRowHalfMirror, 0xF, 0xF, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppRowMirror, 0xF, 0xF, false));
+  return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+             max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
+
+// Sum of an int over the wave, likewise.
+__device__ __forceinline__ int wave_sum_i(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, kDppQuadXor1, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, kDppQuadXor2, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, kDppRowHalfMirror, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, kDppRowMirror, 0xF, 0xF, false);
+  return __builtin_amdgcn_readlane(x, 0) + __builtin_amdgcn_readlane(x, 16) +
+         __builtin_amdgcn_readlane(x, 32) + __builtin_amdgcn_readlane(x, 48);
 }
 
 // Log-sum-exp merge of one (row, q head)'s split partials by one wave, for

@@ -87,17 +87,6 @@ __device__ __forceinline__ typename Vec<T, VEC>::raw_t load_kv(const T* p) {
   return load_raw_stream<T, VEC>(p);
 }
 
-// Maximum of an int over the wave: DPP within rows of 16 lanes, then the 4
-// row results through scalar reads (no LDS traffic).
-__device__ __forceinline__ int wave_max_i(int x) {
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppQuadXor1, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppQuadXor2, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppRowHalfMirror, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, kDppRowMirror, 0xF, 0xF, false));
-  return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
-             max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
-}
-
 // A wave's online-softmax state in LDS (one lane's values 64 floats apart).
 template <int HPW, int VEC>
 __device__ __forceinline__ void store_state(float* lds, int lane, const float (&m)[HPW],

@@ -55,6 +55,10 @@ constexpr int kMinRun = 8;                 // sub-blocks of the shortest key spl
 // of the lengths on the device: 9 prompts of 34-251 queries beside decode rows of up
 // to 4096 tokens (14 sub-blocks, head_dim 64) took 38 us split, 32 whole.
 constexpr int kMinSaved = 12;
+// ... of several sequences: their tiles' partials are more (4 chunks of 200 queries
+// after 256 keys 41.5 us split, 37.4 whole; after 512 41.8 and 44.6; 6 chunks of 300
+// after 512 56.2 and 53.8, after 768 60.5 and 61.4).
+constexpr int kMinSavedBatch = 20;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
@@ -181,15 +185,14 @@ __device__ __forceinline__ Batch rank_batch(const PrefillArgs& a) {
     // Distinct keys: one compare per pair below.
     key = (b.q_len > a.skip_q ? min(b.n, (1 << 24) - 1) + 1 : 0) * 64 + 63 - lane;
   }
-  const int mine = min(b.tiles * (max(0, b.n - b.q_len / 2) / kSB + 1), 1 << 24);
+  b.all_tiles = wave_sum_i(b.tiles);
+  b.work = wave_sum_i(min(b.tiles * (max(0, b.n - b.q_len / 2) / kSB + 1), 1 << 24));
+  b.longest = wave_max_i(b.tiles > 0 ? b.n / kSB + 1 : 0);
   for (int j = 0; j < (int)a.num_seqs; ++j) {
     const bool ahead = __builtin_amdgcn_readlane(key, j) > key;
     const int tiles = __builtin_amdgcn_readlane(b.tiles, j);
     b.rank += ahead;
     b.before += ahead ? tiles : 0;
-    b.all_tiles += tiles;
-    b.work += __builtin_amdgcn_readlane(mine, j);
-    b.longest = max(b.longest, tiles > 0 ? __builtin_amdgcn_readlane(b.n, j) / kSB + 1 : 0);
   }
   return b;
 }
@@ -202,15 +205,16 @@ __device__ __forceinline__ Batch rank_batch(const PrefillArgs& a) {
 // the runs aim at one full residency of the chip: 512 queries after 6656 keys
 // (16 x 128 heads, 64 tiles) 194 us unsplit, 61 / 56 / 55 / 62 us aiming at 384 /
 // 512 / 768 / 1024 workgroups. Past that the partials cost more than they save
-// (66 KB written and read per workgroup; 6 us of write and a 10 us merge here).
+// (66,560 bytes written and read per workgroup; 6 us of write and a 10 us merge here).
 __device__ __forceinline__ int split_run(const Batch& b, const PrefillArgs& a) {
   // A tile's last run is shorter: leave room for one such run per tile.
   const int items = max(a.target - b.all_tiles * a.kv_heads, a.target / 4);
   const int even = (int)min(((int64_t)b.work * a.kv_heads + items - 1) / items, (int64_t)1 << 24);
   const int run = max(max(kMinRun, even), ceil_div(b.longest, a.splits));
-  // The host's test (kMinSaved) with the tiles and lengths that the batch has.
+  // The host's test (most_splits) with the tiles and lengths that the batch has.
   const int idle = a.target - b.all_tiles * a.kv_heads;
-  return (int64_t)b.longest * idle < (int64_t)kMinSaved * a.target ? max(run, b.longest) : run;
+  const int saved = a.num_seqs > 1 ? kMinSavedBatch : kMinSaved;
+  return (int64_t)b.longest * idle < (int64_t)saved * a.target ? max(run, b.longest) : run;
 }
 
 // Page addressing modes: kDiv (any block size), kShift (power of two).
@@ -904,13 +908,14 @@ extern "C" size_t vrh_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t ma
 // depends on shapes only (graph capture): the tiles are estimated from total_q
 // (a ragged sequence fills half of its last tile on average) and the longest
 // context from the table width; the kernel then sizes the runs from the device
-// lengths (split_plan).
+// lengths (split_run).
 namespace {
 // Workgroups the splits aim at: those the chip holds at once (256 CUs, three
-// per CU by registers and LDS at head_dim 96 and 128, four at 64 and 32).
+// per CU by registers and LDS at head_dim 96 and 128, four at 64; at 32, where five
+// would fit, also four).
 constexpr int kCus = 256;
 int target_items(int32_t head_dim) { return kCus * (head_dim <= 64 ? 4 : kWgPerCu); }
-constexpr int kMaxSlots = 1536;     // partials held (68 KB each at head_dim 128)
+constexpr int kMaxSlots = 1536;     // partials held (66,560 bytes each at head_dim 128)
 constexpr int kMaxKeySplits = 16;
 // Head dims of the MFMA tiles (16-bit types, 16-byte aligned rows).
 bool tile_head_dim(int32_t head_dim) { return head_dim >= 32 && head_dim <= 128 && head_dim % 32 == 0; }
@@ -936,7 +941,8 @@ int32_t most_splits(int64_t num_seqs, int64_t total_q, int32_t max_seqlen_q, int
       std::min(most, (total_q * group + num_seqs * kBM / 2) / kBM * kv_heads);
   const int64_t nsub = ceil_div64((int64_t)table_width * block_size, kSB);
   const int64_t target = target_items(head_dim);
-  if (est >= target || nsub * (target - est) < kMinSaved * target) return 1;
+  const int saved = num_seqs > 1 ? kMinSavedBatch : kMinSaved;
+  if (est >= target || nsub * (target - est) < saved * target) return 1;
   return (int32_t)std::max<int64_t>(
       1, std::min({(int64_t)kMaxKeySplits, kMaxSlots / most, ceil_div64(nsub, kMinRun)}));
 }
