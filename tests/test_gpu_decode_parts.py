@@ -48,7 +48,7 @@ def parts(n, block, window, dtype, head_dim, per_wave):
     pages = -(-n // block) - start // block
     least = shortest if long < pages <= constant("kShortSplits") * shortest else long
     split = max(least, -(-pages // 16))
-    if split < 4 * shortest:
+    if split <= 4 * shortest:
         return 1
     lanes = 1
     while lanes * 16 // size < head_dim:
@@ -82,10 +82,12 @@ def test_parts_side_by_side_equal_parts_in_turn(gpu, dtype, heads, kv_heads, hea
     repeat = 1 + -(-constant("kWideGroupSplits") // (16 * kv_heads) // len(lengths)) * 2
     index = torch.arange(len(lengths), device=gpu).repeat(repeat)
     many = paged_attention(q[index], k, v, tables[index].contiguous(), context[index], window)
+    few = paged_attention(q, k, v, tables, context, window)
     expected = oracle_decode(q, k, v, tables, context, window)
     for row in range(len(lengths)):
         alone = paged_attention(q[row : row + 1], k, v, tables[row : row + 1].contiguous(),
                                 context[row : row + 1], window)
+        assert torch.equal(alone[0], few[row]), row
         assert torch.equal(alone[0], many[row]), row
         assert torch.equal(alone[0], many[len(lengths) * (repeat - 1) + row]), row
         assert_close(alone, expected[row : row + 1], dtype)

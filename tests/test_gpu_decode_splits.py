@@ -45,7 +45,8 @@ def expected_splits(n, short, block=16):
 
 @pytest.mark.parametrize("dtype,heads,kv_heads,head_dim,short", [
     (torch.bfloat16, 2, 2, 128, 64), (torch.float32, 2, 2, 128, 32), (torch.float16, 2, 2, 64, 128),
-    (torch.float16, 4, 1, 128, 64), (torch.bfloat16, 8, 1, 128, 64)])
+    (torch.float16, 4, 1, 128, 128), (torch.bfloat16, 8, 1, 128, 128),  # grouped: no short ones
+    (torch.float32, 8, 1, 128, 128)])
 @pytest.mark.parametrize("wider", [0, 200])
 def test_splits_follow_the_row_length(gpu, dtype, heads, kv_heads, head_dim, short, wider):
     long = min(128, 2 * short)

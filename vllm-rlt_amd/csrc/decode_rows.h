@@ -68,14 +68,14 @@ __device__ __forceinline__ Partition partition(int n, const DecodeArgs& a) {
   return p;
 }
 
-// Pages per part of a split (the whole split: one part). A split shorter than two
+// Pages per part of a split (the whole split: one part). A split of up to two
 // shortest parts is not cut: folding costs launches that run parts in turn 4-8 % at
 // two parts (6 rows of 2300-3000 tokens, 32 over 8 heads, 27.2 against 25.6 us) and
-// gains lone rows little (19.8 against 21.5). Parts are whole chunks, so that only a
-// split's last one has a chunk that is not full (3 rows of 18000-22500 tokens 97.9
-// us without, 94.2 with).
+// gains lone rows little (19.8 against 21.5; tables of up to 4096 tokens then have no
+// parts at all). Parts are whole chunks, so that only a split's last one has a chunk
+// that is not full (3 rows of 18000-22500 tokens 97.9 us without, 94.2 with).
 __device__ __forceinline__ int part_pages(const Partition& p, const DecodeArgs& a) {
-  if (p.bps < 2 * a.min_part) return p.bps;
+  if (p.bps <= 2 * a.min_part) return p.bps;
   const int even = ceil_div(p.bps, a.max_parts);
   return max(a.min_part, ceil_div(even, a.part_unit) * a.part_unit);
 }

@@ -49,16 +49,17 @@ namespace {
 
 // K bytes of the shortest splits (64 tokens of a 16-bit type at head_dim 128, 32 of
 // fp32), at most kSplitTokens tokens (shorter ones of head_dim 64: 18 rows of up
-// to 1757 tokens over 8 kv heads 32 against 24 us). Rows of two to kShortSplits of
-// them are cut that finely; shorter rows are one split (64 bf16 rows of 65-128
-// tokens 11.6 us, 16.0 in two splits and a merge), longer ones have splits twice as
-// long (up to kSplitTokens). Against 128 tokens in every row: 8 fp32 rows of 64-512
-// tokens 13.8 against 19.1 us, 64 bf16 rows of 64-512 33.5 against 36.8, 8 of
-// 512-1000 15.2 against 15.5. With up to 16 short splits: 128 rows sharing 512
-// tokens 141 us, 135 with 6; 37 rows of 64-1500, 64 over 8 heads, 32.5 and 28.1;
-// with 8: 8 bf16 rows of 512-1000 15.8; with 4: 100 rows of 16-300 39.3 and 31.5.
-// What the fine splits cost: 64 fp32 rows of 65-128 tokens 23.7 us, 20.1 as one
-// split (in which the 8 fp32 rows above would take 21).
+// to 1757 tokens over 8 kv heads 32 against 24 us). Without grouping, rows of two to
+// kShortSplits of them are cut that finely; shorter rows are one split (64 bf16 rows
+// of 65-128 tokens 11.6 us, 16.0 in two splits and a merge), longer ones have splits
+// twice as long (up to kSplitTokens). Against 128 tokens in every row: 8 fp32 rows of
+// 64-512 tokens 14.4 against 19.1 us, 64 bf16 rows of 64-512 33.5 against 36.8, one of
+// 300 9.2 against 11.9. With up to 16 short splits: 128 rows sharing 512 tokens 141
+// us, 135 with 6; with 8: 8 bf16 rows of 512-1000 15.8, 15.2 with 6; with 4: 64 rows
+// of 64-512 36.4. What the fine splits cost: 64 fp32 rows of 65-128 tokens 23.7 us,
+// 20.1 as one split (in which the 8 fp32 rows above would take 21). Grouped heads
+// have kSplitTokens in every row: 64 rows of 64-512, 32 over 8 heads, 28.3 us, 32.3
+// with fine splits (one row of 300 18.2 and 13.0).
 constexpr int kShortSplits = 6;
 constexpr int kSplitBytes = 16384;
 constexpr int kSplitTokens = 128;
@@ -517,13 +518,14 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
 // fp32, at 768 (3 rows of 24000 tokens) 79.4 / 147 us against 82.8 / 158 in turn, at
 // 1024 (4 rows of 3000) 25.4 / 33.7 against 21.0 / 32.5. Several heads: four parts
 // at 1536 (12 rows of 24000, 32 over 8 heads) 171 against 197, at 2048 (16 rows of
-// 18000-24000) 274 against 248; with two parts two of the four waves idle (6 rows of
-// 3000, 768 splits, 36 against 27). Eight heads per wave, 16 over 2 of dim 32: 6
+// 18000-24000) 274 against 248; with fewer parts some of the four waves idle (6 rows
+// of 3000, 768 splits, two parts: 36 against 27; 11 rows of 9300, head_dim 64, 1408
+// splits, three: 67 against 52). Eight heads per wave, 16 over 2 of dim 32: 6
 // rows of 24000 (768) 85 against 76. MFMA kernel (8 kv heads): 6 rows of 24000
 // (768) 108 against 124, 8 rows of 8000 (1024) 49 against 46.
 constexpr int kWideSplits = 768;
 constexpr int kWideMfmaSplits = 768;
-constexpr int kWideGroupSplits = 1536;  // two or four heads per wave, more than two parts
+constexpr int kWideGroupSplits = 1536;  // two or four heads per wave, four parts
 constexpr int kWideFewSplits = 512;     // otherwise
 
 // Grid form: one wave per (split column, group of HPW q heads, row).
@@ -1080,7 +1082,6 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   a.num_seqs = num_seqs;
   a.expand_e = expand_e;
   a.q_heads = q_heads;
-  a.group = q_heads / kv_heads;
   a.head_dim = head_dim;
   a.block_size = block_size;
   a.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
@@ -1093,8 +1094,10 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   const int split_tokens = std::min(kSplitTokens, kSplitBytes / (head_dim * es));
   a.min_bps = workspace != nullptr ? std::max(1, split_tokens / block_size)
                                    : std::max(1, table_width);
-  a.short_pages = workspace != nullptr ? kShortSplits * a.min_bps : 0;
-  a.long_bps = std::max(a.min_bps, std::min(kSplitTokens, 2 * split_tokens) / block_size);
+  a.group = q_heads / kv_heads;
+  a.short_pages = workspace != nullptr && a.group == 1 ? kShortSplits * a.min_bps : 0;
+  const int long_tokens = a.group == 1 ? std::min(kSplitTokens, 2 * split_tokens) : kSplitTokens;
+  a.long_bps = std::max(a.min_bps, long_tokens / block_size);
 
   // Grouped-query heads per wave: the largest of 8, 4, 2 dividing the group
   // (1 without grouping, or where no grouped instantiation exists).
@@ -1119,11 +1122,14 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
   a.max_parts = mfma_gqa || hpw > 1 ? kGroupParts : kParts;
   const int chunk = mfma_gqa ? kMfmaChunk : std::min(kU, std::max(1, 2 * kU / hpw)) * (64 / lpt);
   a.part_unit = std::max(1, chunk / block_size);
-  // Largest split count any row of this table width can need: the grid is a
-  // function of shapes only (graph capture), never of device lengths.
-  const int max_pages = std::max(1, table_width);
-  // No more columns than that: 37 rows of 64-900 tokens over 8 kv heads, splits of
-  // 128 tokens, 35 us with 16 columns and 28 with 8.
+  // Largest split count any row of this table width (and window) can need: the grid
+  // is a function of shapes only (graph capture), never of device lengths. No more
+  // columns than that: 37 rows of 64-900 tokens over 8 kv heads, splits of 128 tokens,
+  // 35 us with 16 columns and 28 with 8; 19 rows with a window of 569 under a table of
+  // 33792 tokens 34.6 us with 16 and 20.4 with 5.
+  const int max_pages =
+      std::max<int64_t>(1, window > 0 ? std::min<int64_t>(table_width, (int64_t)window / block_size + 2)
+                                      : table_width);
   const int gx = std::min(
       kMaxSplits,
       std::max(max_pages > a.long_bps ? ceil_div(std::min(max_pages, a.short_pages), a.min_bps) : 1,
@@ -1135,19 +1141,17 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
     a.row_base = first;
     const unsigned count = (unsigned)std::min<int64_t>(rows - first, kRowsPerLaunch);
     bool ok = false;
-    // Splits of rows this table (and window) could hold: how many parts they can
-    // have, and whether each gets a workgroup (kWideSplits).
-    const int seen_pages =
-        window > 0 ? (int)std::min<int64_t>(max_pages, (int64_t)window / block_size + 2) : max_pages;
-    const int longest = std::max(a.long_bps, ceil_div(seen_pages, kMaxSplits));
-    const int parts = longest < 2 * a.min_part
+    // How many parts the splits of such rows can have, and whether each split gets a
+    // workgroup (kWideSplits).
+    const int longest = std::max(a.long_bps, ceil_div(max_pages, kMaxSplits));
+    const int parts = longest <= 2 * a.min_part
                           ? 1
                           : std::min(a.max_parts, ceil_div(longest, a.min_part));
     const int units = mfma_gqa ? kv_heads : q_heads / hpw;
-    const int widest = mfma_gqa               ? kWideMfmaSplits
-                       : hpw == 1             ? kWideSplits
-                       : hpw < 8 && parts > 2 ? kWideGroupSplits
-                                              : kWideFewSplits;
+    const int widest = mfma_gqa                          ? kWideMfmaSplits
+                       : hpw == 1                        ? kWideSplits
+                       : hpw < 8 && parts == kGroupParts ? kWideGroupSplits
+                                                         : kWideFewSplits;
     const bool wide = parts > 1 && (int64_t)gx * units * count <= widest;
     const int waves = parts <= 1 ? 0 : !wide ? 1 : parts > 4 ? 8 : 4;
     const dim3 grid((unsigned)gx, (unsigned)units, count);
