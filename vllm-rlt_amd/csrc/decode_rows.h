@@ -35,6 +35,7 @@ struct DecodeArgs {
   const int32_t* cu_q;
   int32_t num_seqs;
   int32_t expand_e;
+  int32_t unit_group;  // waves (or workgroups) of one kv head, split and row
   int32_t q_heads, group, head_dim, block_size, bs_shift, window, min_bps, table_width;
   int32_t long_bps;   // pages of the shortest split of other rows
   int32_t short_pages;  // longest row (pages) cut into splits of min_bps
