@@ -36,7 +36,6 @@ struct DecodeArgs {
   int32_t num_seqs;
   int32_t expand_e;
   int32_t unit_group;  // waves (or workgroups) of one kv head, split and row
-  int32_t wide_units, wide_rows;  // of a launch with a workgroup of several waves per split
   int32_t q_heads, group, head_dim, block_size, bs_shift, window, min_bps, table_width;
   int32_t long_bps;   // pages of the shortest split of other rows
   int32_t short_pages;  // longest row (pages) cut into splits of min_bps

@@ -458,27 +458,10 @@ __device__ __forceinline__ void decode_work(const DecodeArgs& a, int64_t row, in
   run(std::false_type{});
 }
 
-// Grid slot of this wave: its row (after the longest-first ranking), its unit (the
-// heads it serves) and its first split. False when the slot has no row. The grid is
-// (split, unit, row), the split rotated. Where each split has a workgroup of several
-// waves the grid is flat and the split slowest: few such workgroups are resident at
-// once, and the low splits, which every row has, must not wait behind empty ones (2
-// rows of 70-117 tokens, 16 heads of dim 64, under a table of 33792 tokens 9.8 us with
-// the splits fastest, 8.1). There each split starts one (row, unit) further, which
-// spreads a row's splits over the XCDs.
-template <bool kWide>
-__device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int& unit,
-                                          int& split0) {
-  unsigned slot_row = blockIdx.z;
-  unit = (int)blockIdx.y;
-  if constexpr (kWide) {
-    const unsigned per_split = (unsigned)(a.wide_units * a.wide_rows);
-    split0 = (int)(blockIdx.x / per_split);
-    const unsigned at = blockIdx.x % per_split + split0;
-    slot_row = at % per_split / a.wide_units;
-    unit = (int)(at % per_split % a.wide_units);
-  }
-  row = a.row_base + slot_row;
+// Grid slot of this wave: its row (after the longest-first ranking) and its
+// first split (rotated). False when the slot has no row.
+__device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int& split0) {
+  row = a.row_base + blockIdx.z;
   // Longest splits first: within each group of 64 consecutive rows, grid
   // row slot z takes the row of rank z by split length (pages per split,
   // descending; ties keep row order, so rows whose splits are equally long,
@@ -489,14 +472,14 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
   // when the split lengths differ), so no extra launch is needed.
   if (a.cu_q == nullptr) {
     const int lane = threadIdx.x & 63;
-    const int64_t g0 = row - (slot_row & 63);
+    const int64_t g0 = row - (blockIdx.z & 63);
     const int64_t mine = g0 + lane;
     int key = -1;
     if (mine < a.rows) {
       const int n = clamp_length(a.lengths[mine], a);
       key = n > 0 ? max(partition(n, a).bps, a.long_bps) : 0;
     }
-    const int slot = (int)(slot_row & 63);
+    const int slot = (int)(blockIdx.z & 63);
     // Rank only when the group's split lengths differ by 2x or more: only then
     // does the order shorten the drain (and rows of equal split length, such
     // as rows sharing a prefix, keep their dispatch neighbourhood). The short
@@ -521,7 +504,6 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
       row = g0 + __builtin_ffsll((long long)hit) - 1;
     }
   }
-  if constexpr (kWide) return true;
   // Workgroup L = x + gx * (unit + units * row) runs on XCD L % 8. Rows need
   // different split counts, so with split = x the low split indices (present
   // in every row) would pile onto the same XCDs; rotating the split index by
@@ -562,10 +544,9 @@ void paged_decode_kernel(DecodeArgs a) {
   constexpr int kSlots = WAVES > 1 ? WAVES - 1 : WAVES;
   __shared__ float state[kSlots > 0 ? kSlots * HPW * (VEC + 2) * 64 : 1];
   int64_t row;
-  int unit, split0;
-  if (!grid_slot<(WAVES > 1)>(a, row, unit, split0)) return;
-  decode_work<T, VEC, LPT, HPW, WAVES>(a, row, unit * HPW, split0,
-                                       WAVES > 1 ? kMaxSplits : (int)gridDim.x, state);
+  int split0;
+  if (!grid_slot(a, row, split0)) return;
+  decode_work<T, VEC, LPT, HPW, WAVES>(a, row, (int)blockIdx.y * HPW, split0, gridDim.x, state);
 }
 
 // ------------------------------------------------ grouped-query heads on MFMA
@@ -902,10 +883,9 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t vt[WAVES > 1 ? WAVES : 1][kMfmaChunk * D];
   extern __shared__ float mfma_state[];
   int64_t row;
-  int unit, split0;
-  if (!grid_slot<(WAVES > 1)>(a, row, unit, split0)) return;
-  decode_work_mfma<T, D, WAVES>(a, row, unit * a.group, split0,
-                                WAVES > 1 ? kMaxSplits : (int)gridDim.x,
+  int split0;
+  if (!grid_slot(a, row, split0)) return;
+  decode_work_mfma<T, D, WAVES>(a, row, (int)blockIdx.y * a.group, split0, gridDim.x,
                                 vt[WAVES > 1 ? threadIdx.x >> 6 : 0], mfma_state);
 }
 
@@ -1184,10 +1164,7 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
                                                          : kWideFewSplits;
     const bool wide = parts > 1 && (int64_t)gx * units * count <= widest;
     const int waves = parts <= 1 ? 0 : !wide ? 1 : parts > 4 ? 8 : 4;
-    a.wide_units = units;
-    a.wide_rows = (int32_t)count;
-    const dim3 grid = wide ? dim3((unsigned)gx * units * count)
-                           : dim3((unsigned)gx, (unsigned)units, count);
+    const dim3 grid((unsigned)gx, (unsigned)units, count);
     if (mfma_gqa) {
       ok = true;
       if (dtype == VRH_DTYPE_BF16) {
