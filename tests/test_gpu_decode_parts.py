@@ -78,8 +78,8 @@ def test_parts_side_by_side_equal_parts_in_turn(gpu, dtype, heads, kv_heads, hea
 
     q, k, v, tables, context = random_paged(list(lengths), heads, kv_heads, head_dim, dtype, gpu,
                                             block=block, seed=sum(lengths))
-    # Over 1536 splits in one launch: each row many times over.
-    repeat = 1 + -(-constant("kWideGroupSplits") // (16 * kv_heads) // len(lengths)) * 2
+    # More workgroups than are resident at once: each row many times over.
+    repeat = 1 + -(-3 * constant("kCus") // (16 * kv_heads) // len(lengths)) * 2
     index = torch.arange(len(lengths), device=gpu).repeat(repeat)
     many = paged_attention(q[index], k, v, tables[index].contiguous(), context[index], window)
     few = paged_attention(q, k, v, tables, context, window)

@@ -522,20 +522,20 @@ __device__ __forceinline__ bool grid_slot(const DecodeArgs& a, int64_t& row, int
   return true;
 }
 
-// Splits of a launch up to which each split gets a workgroup, one wave a part:
-// with more, single waves fill the chip by themselves. One head per wave, bf16 /
-// fp32, at 768 (3 rows of 24000 tokens) 79.4 / 147 us against 82.8 / 158 in turn, at
-// 1024 (4 rows of 3000) 25.4 / 33.7 against 21.0 / 32.5. Several heads: four parts
-// at 1536 (12 rows of 24000, 32 over 8 heads) 171 against 197, at 2048 (16 rows of
-// 18000-24000) 274 against 248; with fewer parts some of the four waves idle (6 rows
-// of 3000, 768 splits, two parts: 36 against 27; 11 rows of 9300, head_dim 64, 1408
-// splits, three: 67 against 52). Eight heads per wave, 16 over 2 of dim 32: 6
-// rows of 24000 (768) 85 against 76. MFMA kernel (8 kv heads): 6 rows of 24000
-// (768) 108 against 124, 8 rows of 8000 (1024) 49 against 46.
-constexpr int kWideSplits = 768;
-constexpr int kWideMfmaSplits = 768;
-constexpr int kWideGroupSplits = 1536;  // two or four heads per wave, four parts
-constexpr int kWideFewSplits = 512;     // otherwise
+// Splits of a launch up to which each split gets a workgroup, one wave a part: as
+// many workgroups as are resident at once, by registers (one of eight waves to a CU,
+// three of four waves with one head, two with several; three in the MFMA kernel, by
+// LDS two for groups of more than 12 at head_dim 128).
+// Only the device knows how long the rows are: under a wide table most of them may
+// have splits of one part, which one wave of the workgroup runs while the others hold
+// their registers, and a second round of such workgroups doubles the call (12 rows of
+// 500-4000 tokens, 32 over 8 heads, table of 33792: 64 us at 1536 workgroups, 36 with
+// parts in turn; 2 rows, 16 heads, 36 and 21 at 512 of eight waves). Within one round
+// such rows lose up to 11 % (3 rows, 64 over 8 heads, 18.7 and 16.8) and long ones
+// gain 1.5 to 3 times: one row of 24000 tokens 32 against 63 us, 4 rows, 32 over 8
+// heads, 61 against 121, 6 rows, 64 over 8 heads, 108 against 124.
+constexpr int kCus = 256;
+constexpr int kWideParts = 4;  // parts of a workgroup of four waves
 
 // Grid form: one wave per (split column, group of HPW q heads, row).
 template <typename T, int VEC, int LPT, int HPW, int WAVES>
@@ -1151,19 +1151,20 @@ int vrh_decode_rows(int dtype, void* out, const void* q, const void* key_cache,
     const unsigned count = (unsigned)std::min<int64_t>(rows - first, kRowsPerLaunch);
     bool ok = false;
     // How many parts the splits of such rows can have, and whether each split gets a
-    // workgroup (kWideSplits).
+    // workgroup.
     const int longest = std::max(a.long_bps, ceil_div(max_pages, kMaxSplits));
     const int parts = longest <= 2 * a.min_part
                           ? 1
                           : std::min(a.max_parts, ceil_div(longest, a.min_part));
     const int units = mfma_gqa ? kv_heads : q_heads / hpw;
     a.unit_group = units / kv_heads;
-    const int widest = mfma_gqa                          ? kWideMfmaSplits
-                       : hpw == 1                        ? kWideSplits
-                       : hpw < 8 && parts == kGroupParts ? kWideGroupSplits
-                                                         : kWideFewSplits;
-    const bool wide = parts > 1 && (int64_t)gx * units * count <= widest;
-    const int waves = parts <= 1 ? 0 : !wide ? 1 : parts > 4 ? 8 : 4;
+    const size_t mfma_lds = kWideParts * (size_t)kMfmaChunk * head_dim * 2 +
+                            (kWideParts - 1) * mfma_state_bytes(head_dim, a.group);
+    const int per_cu = mfma_gqa  ? std::min(3, (int)(160 * 1024 / mfma_lds))
+                       : hpw > 1 ? 2
+                                 : parts > kWideParts ? 1 : 3;
+    const bool wide = parts > 1 && (int64_t)gx * units * count <= per_cu * kCus;
+    const int waves = parts <= 1 ? 0 : !wide ? 1 : parts > kWideParts ? 8 : 4;
     const dim3 grid((unsigned)gx, (unsigned)units, count);
     if (mfma_gqa) {
       ok = true;
