@@ -786,7 +786,7 @@ def main():
 
     if not args.skip_extras:
         # Eager step: the 24 layer calls launched from Python through the
-        # ctypes boundary (host argument marshalling included), for comparison
+        # adapter boundary (host argument handling included), for comparison
         # with the graph-replayed step above.
         eager_ms = event_time_ms(eager_step, 20)
         # The same step through the registered torch op (vllm_rlt._C), and the
@@ -801,7 +801,7 @@ def main():
 
         eager_op_ms = event_time_ms(eager_op_step, 20)
         host_us = {}
-        for name, fn in (("ctypes", eager_step), ("torch_op", eager_op_step)):
+        for name, fn in (("adapter", eager_step), ("torch_op", eager_op_step)):
             torch.cuda.synchronize()
             t_host = time.perf_counter()
             for _ in range(4):

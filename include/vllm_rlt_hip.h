@@ -185,9 +185,12 @@ size_t vrh_paged_prefill_workspace_bytes(int64_t num_seqs, int32_t max_seqlen_q,
  * leave the GPU partly idle (one prompt chunk, a few short ones) cuts each
  * tile's keys into up to 16 runs computed side by side and merges their fp32
  * partials. A call given at least this many bytes does so; with fewer, down to
- * vrh_paged_prefill_workspace_bytes, it runs one workgroup per tile. The number
- * of runs follows from the call's shapes and lengths, so a query's last bits
- * may differ between batches. */
+ * vrh_paged_prefill_workspace_bytes, it runs one workgroup per tile. The room
+ * follows from the shapes alone (the table's width bounds the contexts): at most
+ * 1536 partials, 97.5 MiB at head_dim 128; none for head dims without MFMA tiles.
+ * Whether and into how many runs a tile is cut follows from the shapes and the
+ * lengths of the whole batch, so a query's last bits may differ between batches;
+ * with the smaller workspace they do not. */
 size_t vrh_paged_prefill_split_workspace_bytes(int64_t num_seqs, int64_t total_q,
                                                int32_t max_seqlen_q, int32_t q_heads,
                                                int32_t kv_heads, int32_t head_dim,

@@ -5,8 +5,8 @@ speculative verification, worker/speculative.py:176-178).
 A packed call whose sequences all have at most 8 queries (max_seqlen_q <= 8)
 runs every query as a split-KV decode row; query i of sequence s must equal,
 with ``torch.equal``, the decode of a row with the same q, the same table row
-and length n_s - q_s + i + 1. Lengths span the decode's 128-token split
-boundaries and its one-split / multi-split cases; values are also checked
+and length n_s - q_s + i + 1. Lengths span the decode's split boundaries (multiples
+of 64 or 128 tokens, 32 or 64 in fp32) and its one-split / multi-split cases; values are also checked
 against the oracle so that equality is not agreement on a wrong answer.
 """
 
@@ -58,7 +58,7 @@ def serial_rows(tables, lengths, cu):
 
 
 CASES = [
-    # (q_lens, context lengths): split boundaries at 128-token multiples,
+    # (q_lens, context lengths): split boundaries at 64- and 128-token multiples,
     # one-split rows, 16-split rows, q_len 1..8
     ([1, 2, 3, 4, 5, 6, 7, 8], [8, 127, 129, 256, 260, 1000, 2049, 4100]),
     ([8] * 6 + [1] * 4, [8, 135, 136, 137, 2055, 3000, 1, 129, 128, 4096]),
